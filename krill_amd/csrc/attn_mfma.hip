@@ -1,6 +1,6 @@
-// Paged int8 attention with MFMA tiles: the speculative-verify / chunked-
-// prefill path, used when a KV head serves more than 8 query rows
-// (GQA group x new tokens).  Reference semantics: the same SDPA call with
+// Paged int8 attention with MFMA tiles: the speculative-verify path, used
+// when a KV head serves 9 to 64 query rows (GQA group x new tokens; longer
+// windows: attn_prefill.hip).  Reference semantics: the same SDPA call with
 // L > 1 new rows and the block-causal mask of
 // Sources/KrillEngine/BatchedDecode.swift:299-312 (row j of the new window
 // sees every cached key plus new keys 0..j), equivalently
@@ -54,12 +54,6 @@ __host__ __device__ constexpr int mfma_stages(int D, int G, int W) {
   return W > 1 && 3 * mfma_stage_bytes(D, G) * (8 / W) <= 160 * 1024 ? 3 : 2;
 }
 
-// Two waves per SIMD for the 32-row, 4-wave, 128-d affine shape (chunked
-// prefill): left alone the register allocator lands a few registers past
-// the 256 that two waves may hold and the occupancy halves.
-template <int D, int MODE, int NRT, int W>
-constexpr int mfma_min_waves() { return D == 128 && MODE == MODE_AFFINE && NRT == 2 && W == 4 ? 2 : 1; }
-
 // VAR: 0 plain; 1 RoPE of the queries; 2 sliding window (keys below
 // max(win_start[b], position - window + 1) masked).
 // TS: 1 -- the W waves of a workgroup hold W row groups and every wave
@@ -68,8 +62,7 @@ constexpr int mfma_min_waves() { return D == 128 && MODE == MODE_AFFINE && NRT =
 // its own softmax state), so no byte is converted twice; at each segment
 // end the two states are combined through the ring stage just consumed.
 template <int D, int MODE, int NRT, int VAR, int W, int TS>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(mfma_min_waves<D, MODE, NRT, W>())))
-void k_attn_mfma(AttnArgs a) {
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1))) void k_attn_mfma(AttnArgs a) {
   constexpr bool ROPE = VAR == 1, WIN = VAR == 2;
   constexpr int G = MODE == MODE_AFFINE ? D / 64 : 1;
   constexpr int KS = D / 32;   // 32-d steps of Q.K^T
@@ -77,8 +70,7 @@ void k_attn_mfma(AttnArgs a) {
   constexpr int RR = 16 * NRT; // query rows of this wave
   constexpr int STAGE = mfma_stage_bytes(D, G);
   constexpr int NCH = STAGE / 1024;  // direct loads per block
-  // CVT (four-wave groups, affine, head_dim 128: chunked prefill, the
-  // cascade's prefix pass): the four waves convert each staged block once,
+  // CVT (four-wave groups, affine, head_dim 128): the four waves convert each staged block once,
   // a quarter each, into fp16 K and V^T tiles in LDS that all four read,
   // instead of every wave converting the whole block for its own rows; the
   // tiles take the LDS of the third ring stage
@@ -737,7 +729,7 @@ static hipError_t launch_mfma_w(const AttnArgs &args, dim3 grid, hipStream_t st)
 
 // (nrt, group_waves, token_split) shapes the plan may choose: 16-row waves
 // in workgroups of 1, 2 or 4 row groups, or (D <= 128) a 32-row group split
-// over two waves by tokens, or (D <= 128) 32-row waves in workgroups of 4.
+// over two waves by tokens.
 template <int D, int MODE>
 static hipError_t launch_mfma_dm(const AttnArgs &args, const AttnPlan &p, dim3 grid, hipStream_t st) {
   if (p.token_split == 2) {
@@ -746,14 +738,7 @@ static hipError_t launch_mfma_dm(const AttnArgs &args, const AttnPlan &p, dim3 g
     }
     return hipErrorInvalidValue;
   }
-  if (p.token_split != 1) return hipErrorInvalidValue;
-  if (p.nrt == 2) {
-    if constexpr (D <= 128) {
-      if (p.group_waves == 4) return launch_mfma_w<D, MODE, 2, 4, 1>(args, grid, st);
-    }
-    return hipErrorInvalidValue;
-  }
-  if (p.nrt != 1) return hipErrorInvalidValue;
+  if (p.token_split != 1 || p.nrt != 1) return hipErrorInvalidValue;
   switch (p.group_waves) {
     case 1: return launch_mfma_w<D, MODE, 1, 1, 1>(args, grid, st);
     case 2: return launch_mfma_w<D, MODE, 1, 2, 1>(args, grid, st);
@@ -804,23 +789,20 @@ static int32_t occupancy_mfma_sel(int sel) {
     case 0: return occupancy_mfma<D, MODE, 1, 1, 1>();
     case 1: return occupancy_mfma<D, MODE, 1, 2, 1>();
     case 2: return occupancy_mfma<D, MODE, 1, 4, 1>();
-    case 3:
-      if constexpr (D <= 128) return occupancy_mfma<D, MODE, 2, 2, 2>();
-      return 1;
     default:
-      if constexpr (D <= 128) return occupancy_mfma<D, MODE, 2, 4, 1>();
+      if constexpr (D <= 128) return occupancy_mfma<D, MODE, 2, 2, 2>();
       return 1;
   }
 }
 
-int32_t mfma_groups_per_cu(const PoolGeometry &g, int32_t nrt, int32_t group_waves, int32_t token_split) {
+int32_t mfma_groups_per_cu(const PoolGeometry &g, int32_t group_waves, int32_t token_split) {
   const int dsel = g.D == 64 ? 0 : g.D == 128 ? 1 : 2;
-  const int sel = token_split == 2 ? 3 : nrt == 2 ? 4 : group_waves == 4 ? 2 : group_waves == 2 ? 1 : 0;
+  const int sel = token_split == 2 ? 3 : group_waves == 4 ? 2 : group_waves == 2 ? 1 : 0;
   if (g.num_cus <= 0) {  // host-only pool: the LDS bound (the ring per workgroup, 160 KB per CU)
-    static const int est[3][5] = {{5, 5, 3, 8, 3}, {3, 3, 2, 4, 2}, {1, 1, 1, 1, 1}};
+    static const int est[3][4] = {{5, 5, 3, 8}, {3, 3, 2, 4}, {1, 1, 1, 1}};
     return est[dsel][sel];
   }
-  static int cache[2][3][5] = {};  // [mode][D][shape], filled on first use per process
+  static int cache[2][3][4] = {};  // [mode][D][shape], filled on first use per process
   int &c = cache[g.mode == MODE_AFFINE][dsel][sel];
   if (c == 0) {
     int v;

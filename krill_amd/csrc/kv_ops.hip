@@ -774,6 +774,63 @@ __global__ __launch_bounds__(64) void k_attn_merge_flat(AttnArgs a) {
   merge_slots<D>(a, slot0, last - first + 1, rr, a.rows_per_group, obase);
 }
 
+// The same merge after the long-window kernel, whose thousands of rows make a
+// workgroup per row cost more than the merge itself: one workgroup of four
+// waves per (row group, KV head, sequence), each wave the rows rr = wave,
+// wave + 4, ...  Most leave at once: a range covers whole sequences.
+template <int D>
+__global__ __launch_bounds__(256) void k_attn_merge_rows(AttnArgs a) {
+  constexpr int E = D / 64;
+  const int rg = blockIdx.x, hk = blockIdx.y, b = blockIdx.z;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int RR = a.rows_per_group, nrow = min(RR, a.NR - rg * RR);
+  int s = 0, nb = 0;
+  const int T = flat_total_and_start(a, b, rg, s, nb);
+  int first = 0, n = 0;
+  if (nb > 0) {
+    const int Wt = min(a.waves, T);
+    first = flat_wave_of(s, T, Wt);
+    n = flat_wave_of(s + nb - 1, T, Wt) - first + 1;
+    if (n == 1) return;
+  }
+  const int64_t slot0 = ((int64_t)hk * a.row_groups + rg) * (a.waves + a.B) + first + b;
+  const float2 *ml2 = reinterpret_cast<const float2 *>(a.ws_ml);
+  for (int rr = wid; rr < nrow; rr += 4) {
+    const int64_t obase = out_row_base(a, b, hk, rg * RR + rr, D);
+    float M = -INFINITY, lsum = 0.0f, acc[E];
+    for (int k = lane; k < n; k += 64) M = fmaxf(M, ml2[(slot0 + k) * RR + rr].x);
+    M = uniform_f32(wave_allmax(M));
+#pragma unroll
+    for (int e = 0; e < E; ++e) acc[e] = 0.0f;
+    for (int k0 = 0; k0 < n; k0 += 64) {
+      const int cnt = min(64, n - k0);
+      const float2 ml = lane < cnt ? ml2[(slot0 + k0 + lane) * RR + rr] : float2{-INFINITY, 0.0f};
+      const float w = ml.x != -INFINITY ? fast_exp2(ml.x - M) : 0.0f;
+      lsum += w * ml.y;
+      // four slots' rows in flight (past the last one: its row again, weight 0)
+      for (int k = 0; k < cnt; k += 4) {
+        float o[4][E];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float *op = a.ws_o + ((slot0 + k0 + min(k + j, cnt - 1)) * RR + rr) * (int64_t)D + lane;
+#pragma unroll
+          for (int e = 0; e < E; ++e) o[j][e] = op[64 * e];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float wk = k + j < cnt ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), k + j)) : 0.0f;
+#pragma unroll
+          for (int e = 0; e < E; ++e) acc[e] += wk * o[j][e];
+        }
+      }
+    }
+    const float L = uniform_f32(wave_allsum(lsum));
+    const float inv = (M == -INFINITY || !(L > 0.0f)) ? 0.0f : 1.0f / L;
+#pragma unroll
+    for (int e = 0; e < E; ++e) store_out(a.out, obase + lane + 64 * e, acc[e] * inv, a.out_dtype);
+  }
+}
+
 // Shared-prefix cascade: sequence b's keys are the P shared prefix blocks
 // followed by its own suffix blocks.  The prefix pass attends every
 // sequence's query rows to the prefix once (one virtual sequence of length
@@ -1063,6 +1120,25 @@ hipError_t launch_copy_pairs(const PoolGeometry &g, const CopyPair *pairs, int32
   return hipSuccess;
 }
 
+// Block ranges per (KV head, row-group workgroup) of the long-window kernel,
+// hg such workgroups on a chip that holds `cap`: the first k (rounds of
+// resident workgroups) whose floor(k cap / hg) ranges fill at least 90 % of
+// them, else the fullest of the first eight.
+static int64_t prefill_ranges(int64_t cap, int64_t hg) {
+  int64_t best = 1;
+  double fill = 0.0;
+  const int64_t k0 = (hg + cap - 1) / cap;
+  for (int64_t k = k0; k < k0 + 8 && fill < 0.9; ++k) {
+    const int64_t w = k * cap / hg;
+    const double f = (double)(w * hg) / (double)(k * cap);
+    if (f > fill + 1e-9) {
+      fill = f;
+      best = w;
+    }
+  }
+  return best;
+}
+
 int32_t plan_attention(const PoolGeometry &g, int32_t B, int32_t Hq, int32_t Lq, int32_t max_seq_len,
                        int32_t split_blocks, int32_t path, AttnPlan *plan) {
   if (g.Hkv <= 0 || Hq <= 0 || Hq % g.Hkv != 0 || Lq <= 0 || B < 0 || max_seq_len < 0) return -1;
@@ -1070,12 +1146,16 @@ int32_t plan_attention(const PoolGeometry &g, int32_t B, int32_t Hq, int32_t Lq,
   AttnPlan p{};
   p.NR = R * Lq;
   // head_dim 512: the VALU kernel with each block split over four waves of
-  // 128 dims (the MFMA kernel's LDS ring would hold 70 KB per stage), the
+  // 128 dims (the verify kernel's LDS ring would hold 70 KB per stage), the
   // query rows in groups of at most 8 (the largest divisor of NR up to 8),
-  // one grid row group each
+  // one grid row group each, every group reading all of the cache
   const bool dsplit = g.D > 256;
   if (dsplit && path == 2) return -2;
-  p.use_mfma = !dsplit && (path == 2 || (path == 0 && p.NR > 8));
+  // the long-window kernel from 65 rows per KV head on.  At head_dim 512 that
+  // is 9 row groups of the VALU kernel: 256 new rows over contexts of 700 to
+  // 3000 (2048 rows per KV head) take 145 us against 314 us.
+  p.prefill = p.NR > 64 && (dsplit ? path == 0 && Lq > 1 : path != 1);
+  p.use_mfma = p.prefill || (!dsplit && (path == 2 || (path == 0 && p.NR > 8)));
   if (!p.use_mfma && !dsplit && p.NR > 8) return -2;
   const int32_t nb_max = std::max(1, (max_seq_len + 63) / 64);
   const int64_t tmax = (int64_t)B * nb_max;
@@ -1087,27 +1167,28 @@ int32_t plan_attention(const PoolGeometry &g, int32_t B, int32_t Hq, int32_t Lq,
     // 16-row wave leaves room for two waves per SIMD.
     // 17-32 rows (speculative verify) at D <= 128: one 32-row group per
     // workgroup whose two waves split each block's tokens instead, so no
-    // byte is converted twice.  More than 64 rows at D <= 128 (chunked
-    // prefill): 32-row waves in groups of four, each converted byte feeding
-    // two row tiles, when a batch of max_seq_len sequences gives every
-    // workgroup of that grid at least 16 blocks to stream (the cascade's
-    // shared prefix of 65 blocks does not: its 16-row grid keeps more
-    // workgroups busy).
+    // byte is converted twice.  More than 64 rows (chunked prefill): the
+    // long-window kernel, at D <= 128 with 32-row waves (each LDS read feeds
+    // two row tiles) when a batch of max_seq_len sequences gives every
+    // workgroup of that grid at least 16 blocks to stream: a 3900-row prompt
+    // takes 265 us so against 332 us with 16-row waves, the cascade over a
+    // shared prefix of 65 blocks, whose 16-row grid keeps more workgroups
+    // busy, 67 against 63 us.  head_dim 256 in 32-row waves, one a SIMD: 172
+    // against 166 us (512 rows, window 1024).
     p.token_split = 1;
-    const int64_t grp32 = ((p.NR + 31) / 32 + 3) / 4;
-    const bool rows32 = p.NR > 64 && g.D <= 128 &&
-                        tmax >= 16 * (cus * mfma_groups_per_cu(g, 2, 4, 1) / ((int64_t)g.Hkv * grp32));
-    if (p.NR > 16 && p.NR <= 32 && g.D <= 128) {
+    if (p.prefill) {
+      const int64_t grp32 = ((p.NR + 31) / 32 + 3) / 4;
+      const bool rows32 = g.D <= 128 && tmax >= 16 * (cus * prefill_groups_per_cu(g) / ((int64_t)g.Hkv * grp32));
+      p.nrt = rows32 ? 2 : 1;
+      p.rows_per_group = 16 * p.nrt;
+      p.row_groups = (p.NR + p.rows_per_group - 1) / p.rows_per_group;
+      p.group_waves = 4;
+    } else if (p.NR > 16 && p.NR <= 32 && g.D <= 128) {
       p.nrt = 2;
       p.rows_per_group = 32;
       p.row_groups = 1;
       p.group_waves = 1;
       p.token_split = 2;
-    } else if (rows32) {
-      p.nrt = 2;
-      p.rows_per_group = 32;
-      p.row_groups = (p.NR + 31) / 32;
-      p.group_waves = 4;
     } else {
       p.nrt = 1;
       p.rows_per_group = 16;
@@ -1142,8 +1223,12 @@ int32_t plan_attention(const PoolGeometry &g, int32_t B, int32_t Hq, int32_t Lq,
     waves = (tmax + pw - 1) / pw;
   } else if (p.use_mfma) {
     const int64_t groups = (p.row_groups + p.group_waves - 1) / p.group_waves;
-    waves = std::max<int64_t>(1, cus * mfma_groups_per_cu(g, p.nrt, p.group_waves, p.token_split) /
-                                     ((int64_t)g.Hkv * groups));
+    const int64_t per_cu = p.prefill ? prefill_groups_per_cu(g)
+                                     : mfma_groups_per_cu(g, p.group_waves, p.token_split);
+    const int64_t cap = cus * per_cu, hg = (int64_t)g.Hkv * groups;
+    waves = std::max<int64_t>(1, cap / hg);
+    // (a decode step's workspace stays within the static scratch it had)
+    if (p.prefill && Lq > 1) waves = prefill_ranges(cap, hg);
   } else if (dsplit) {
     // workgroups of 4 waves (one per 128-dim slice)
     const int64_t wg_per_cu = std::max<int32_t>(1, valu_waves_per_cu(g, p.rows_per_group) / (g.D / 128));
@@ -1151,7 +1236,8 @@ int32_t plan_attention(const PoolGeometry &g, int32_t B, int32_t Hq, int32_t Lq,
   } else {
     waves = std::max<int64_t>(1, cus * valu_waves_per_cu(g, p.NR) / g.Hkv);
   }
-  waves = std::max<int64_t>(waves, (tmax + 63) / 64);
+  // (the long-window kernel reloads its table register every 64 blocks)
+  if (!p.prefill) waves = std::max<int64_t>(waves, (tmax + 63) / 64);
   p.split_blocks = split_blocks > 0 ? std::min(split_blocks, 64) : 0;
   p.nb_cap = nb_max;
   p.waves = (int32_t)waves;
@@ -1165,6 +1251,11 @@ hipError_t launch_attn_merge(const PoolGeometry &g, int32_t layer, const AttnLau
                              hipStream_t st) {
   if (a.B == 0) return hipSuccess;
   const AttnArgs args = make_attn_args(g, layer, a, p);
+  if (p.prefill) {
+    const dim3 rows((unsigned)p.row_groups, (unsigned)g.Hkv, (unsigned)a.B);
+    KRILL_DISPATCH_D(g.D, { k_attn_merge_rows<D><<<rows, dim3(256), 0, st>>>(args); });
+    return hipGetLastError();
+  }
   const dim3 grid((unsigned)p.NR, (unsigned)g.Hkv, (unsigned)a.B);
   KRILL_DISPATCH_D(g.D, { k_attn_merge_flat<D><<<grid, dim3(64), 0, st>>>(args); });
   return hipGetLastError();
@@ -1192,6 +1283,13 @@ static hipError_t launch_append_newest(const PoolGeometry &g, int32_t layer, con
   return hipGetLastError();
 }
 
+// The attention kernel the plan chose.
+static hipError_t launch_attn_kernel(const PoolGeometry &g, int32_t layer, const AttnLaunch &a, const AttnPlan &p,
+                                     hipStream_t st) {
+  if (p.prefill) return launch_attn_prefill(g, layer, a, p, st);
+  return p.use_mfma ? launch_attn_mfma(g, layer, a, p, st) : launch_attn_valu(g, layer, a, p, st);
+}
+
 hipError_t launch_attention_shared_prefix(const PoolGeometry &g, int32_t layer, const AttnLaunch &pa,
                                          const AttnPlan &pp, const AttnLaunch &sa, const AttnPlan &sp,
                                          hipStream_t st) {
@@ -1199,13 +1297,13 @@ hipError_t launch_attention_shared_prefix(const PoolGeometry &g, int32_t layer, 
   if (pa.B != 1 || pa.len_const < 0 || pa.causal || !pa.partial_only || !sa.partial_only || sa.Lq != 1 ||
       pa.Lq != sa.B)
     return hipErrorInvalidValue;
-  hipError_t e = pp.use_mfma ? launch_attn_mfma(g, layer, pa, pp, st) : launch_attn_valu(g, layer, pa, pp, st);
+  hipError_t e = launch_attn_kernel(g, layer, pa, pp, st);
   if (e != hipSuccess) return e;
   if (sa.k_new && sp.use_mfma) {  // the newest tokens (in the suffix blocks) before the MFMA suffix pass
     e = launch_append_newest(g, layer, sa, sp, st);
     if (e != hipSuccess) return e;
   }
-  e = sp.use_mfma ? launch_attn_mfma(g, layer, sa, sp, st) : launch_attn_valu(g, layer, sa, sp, st);
+  e = launch_attn_kernel(g, layer, sa, sp, st);
   if (e != hipSuccess) return e;
   const AttnArgs ap = make_attn_args(g, layer, pa, pp), as = make_attn_args(g, layer, sa, sp);
   const dim3 grid((unsigned)ap.R, (unsigned)g.Hkv, (unsigned)sa.B);
@@ -1236,7 +1334,7 @@ hipError_t launch_attention(const PoolGeometry &g, int32_t layer, const AttnLaun
     hipError_t e = launch_append_newest(g, layer, a, p, st);
     if (e != hipSuccess) return e;
   }
-  hipError_t e = p.use_mfma ? launch_attn_mfma(g, layer, a, p, st) : launch_attn_valu(g, layer, a, p, st);
+  hipError_t e = launch_attn_kernel(g, layer, a, p, st);
   if (e != hipSuccess) return e;
   // windowed decode kernel at head_dim <= 256: merged inside its workgroups
   if (!p.use_mfma && a.window > 0 && g.D <= 256) return hipSuccess;

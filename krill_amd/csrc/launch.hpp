@@ -53,7 +53,7 @@ struct AttnLaunch {
 // Splits/rows plan shared by the workspace query and the launch.
 struct AttnPlan {
   int32_t NR;             // query rows per KV head = (Hq/Hkv) * Lq
-  int32_t use_mfma;       // 1 when the MFMA kernel runs
+  int32_t use_mfma;       // 1 when an MFMA kernel runs (attn_mfma.hip or, with prefill, attn_prefill.hip)
   int32_t split_blocks;   // option value: blocks per wave (<= 64), 0 automatic
   int32_t waves;          // workgroups per (KV head, row group): the flat block split
   int32_t nb_cap;         // blocks per sequence covered (from max_seq_len)
@@ -64,6 +64,7 @@ struct AttnPlan {
   int32_t group_waves;    // MFMA: row groups per workgroup, one wave each, sharing one LDS ring (1 on the VALU path)
   int32_t token_split;    // MFMA: 2 = one row group per workgroup, its two waves split each block's tokens; else 1
   size_t ws_bytes;
+  int32_t prefill;        // 1: the long-window kernel of attn_prefill.hip
 };
 
 int32_t plan_attention(const PoolGeometry &g, int32_t B, int32_t Hq, int32_t Lq, int32_t max_seq_len,
@@ -109,10 +110,13 @@ int32_t valu_waves_per_cu(const PoolGeometry &g, int32_t NR);
 // Longest windowed view (tokens) of the decode kernel's per-sequence
 // workgroups (head_dim <= 256; 0 elsewhere).
 int32_t valu_window_limit(const PoolGeometry &g, int32_t NR, bool rope);
-// Resident workgroups per compute unit of the MFMA kernel for (D, nrt,
+// Resident workgroups per compute unit of the MFMA kernel for (D,
 // group_waves, token_split, mode) (bound by its LDS ring or its registers), from the
 // occupancy query on a device pool.
-int32_t mfma_groups_per_cu(const PoolGeometry &g, int32_t nrt, int32_t group_waves, int32_t token_split);
+int32_t mfma_groups_per_cu(const PoolGeometry &g, int32_t group_waves, int32_t token_split);
+
+// Resident workgroups (four waves) per compute unit of the long-window kernel.
+int32_t prefill_groups_per_cu(const PoolGeometry &g);
 
 // Per-wave timestamps of the last decode launch (diagnostic build only).
 int32_t wave_stamps(unsigned long long *host, int32_t max_waves);
@@ -122,6 +126,8 @@ hipError_t launch_attn_valu(const PoolGeometry &g, int32_t layer, const AttnLaun
                             hipStream_t st);
 hipError_t launch_attn_mfma(const PoolGeometry &g, int32_t layer, const AttnLaunch &a, const AttnPlan &p,
                             hipStream_t st);
+hipError_t launch_attn_prefill(const PoolGeometry &g, int32_t layer, const AttnLaunch &a, const AttnPlan &p,
+                               hipStream_t st);
 hipError_t launch_attn_merge(const PoolGeometry &g, int32_t layer, const AttnLaunch &a, const AttnPlan &p,
                              hipStream_t st);
 

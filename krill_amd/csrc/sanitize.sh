@@ -39,7 +39,7 @@ for san in "${SANS[@]}"; do
   "$CXX" -std=c++17 -O1 -g -fPIC -fno-omit-frame-pointer -fsanitize="$san" \
     -c "$HERE/block_manager.cpp" -o "$out/block_manager.o"
   "$CXX" -shared -fPIC --hip-link --offload-arch="$ARCH" -fsanitize="$san" -shared-libsan -o "$out/libkrillhip.so" \
-    "$out/capi.o" "$out/block_manager.o" "$HERE/_build/kv_ops.o" "$HERE/_build/attn_valu.o" "$HERE/_build/attn_mfma.o" "$HERE/_build/scratch.o"
+    "$out/capi.o" "$out/block_manager.o" "$HERE/_build/kv_ops.o" "$HERE/_build/attn_valu.o" "$HERE/_build/attn_mfma.o" "$HERE/_build/attn_prefill.o" "$HERE/_build/scratch.o"
 
   tree="$(mktemp -d)"
   trap 'rm -rf "$tree"' EXIT

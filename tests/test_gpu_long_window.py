@@ -1,0 +1,118 @@
+"""Attention of long query windows (more than 64 rows per KV head): the kernel of
+attn_prefill.hip against the fp64 oracle, at the edges of its row tiles (16 and 32 rows a
+wave, four waves a workgroup), of its 64-key blocks, of its 64-entry table window and of the
+block ranges a workgroup takes.
+
+Bound: bf16 and fp16 inputs reach the matrix cores exactly, the weights as fp16 pairs (2^-22)
+and the sums are binary32, so outputs of values of order 1 lie within 1e-4 of the oracle; 2e-3
+is the bound of the repository's other attention tests."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+import krill_amd  # noqa: E402
+from tests.kvutil import Filled, i32, oracle_attention, rand_bits, to_dev  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+ATOL = 2e-3
+
+
+def _run(mode, D, H, R, lens, Lq, dt="bf16", scale=None, split_blocks=0, out_dtype=torch.float32, q_mul=1.0, seed=0):
+    rng = np.random.default_rng(seed)
+    pool = krill_amd.KVPool(1, H, D, sum((n + 63) // 64 for n in lens) + 4, mode, dt, free_list_seed=7)
+    if split_blocks:
+        pool.set_option(krill_amd._lib.OPT_SPLIT_BLOCKS, split_blocks)
+    f = Filled(pool, lens, rng, dt, max_chunk=500)
+    tables, n, _ = f.tables()
+    scale = 1.0 / np.sqrt(D) if scale is None else scale
+    q = rand_bits(rng, (len(lens), H * R, Lq, D), dt, scale=q_mul)
+    got = pool.attention(0, to_dev(q, dt), tables, n, max(lens), float(scale), out_dtype)
+    torch.cuda.synchronize()
+    ref = oracle_attention(pool, f, 0, q, dt, scale)
+    pool.close()
+    return got.double().cpu().numpy(), ref
+
+
+@pytest.mark.parametrize("mode", ["affine_g64", "ref_row"])
+@pytest.mark.parametrize("D,R,Lq", [(64, 5, 13), (64, 8, 17), (128, 5, 13), (128, 2, 64), (256, 2, 33), (256, 3, 43),
+                                    (512, 8, 9), (512, 1, 65)])
+def test_row_and_block_edges(mode, D, R, Lq):
+    """65 (one row past four 16-row tiles) to 136 rows; sequences ending at, one before and one
+    past a block edge, one holding only its new rows, one empty of older blocks."""
+    print(f"\ncase long_window mode={mode} D={D} R={R} Lq={Lq}", flush=True)
+    got, ref = _run(mode, D, 2, R, [Lq, 127, 128, 129, 300], Lq, dt="f16" if R == 8 else "bf16", seed=D + R)
+    assert np.abs(got - ref).max() <= ATOL
+
+
+@pytest.mark.parametrize("mode", ["affine_g64", "ref_row"])
+@pytest.mark.parametrize("D,split", [(64, 0), (128, 0), (128, 3), (256, 2), (512, 2)])
+def test_ranges_across_sequences(mode, D, split):
+    """Ranges that begin and end inside sequences (partials merged), whole sequences inside one
+    range, and (automatic split, one KV head) ranges over several sequences."""
+    print(f"\ncase long_window_ranges mode={mode} D={D} split={split}", flush=True)
+    got, ref = _run(mode, D, 1, 3, [40, 700, 65, 1300, 64, 90], 33, split_blocks=split, seed=D)
+    assert np.abs(got - ref).max() <= ATOL
+
+
+@pytest.mark.parametrize("mode", ["affine_g64", "ref_row"])
+def test_range_longer_than_the_table_window(mode):
+    """A whole prompt of 72 blocks on 8 KV heads, 108 row-group workgroups each, so many that each
+    takes its rows' whole range: up to 72 blocks, past the 64 table entries a workgroup holds at
+    once.  Checked on rows of the first, a middle and the last blocks against the same rows as a
+    short window."""
+    print(f"\ncase long_window_table mode={mode}", flush=True)
+    H, R, D, T, dt = 8, 3, 128, 72 * 64 - 5, "bf16"
+    rng = np.random.default_rng(3)
+    pool = krill_amd.KVPool(1, H, D, 80, mode, dt, free_list_seed=9)
+    f = Filled(pool, [T], rng, dt, max_chunk=4000)
+    tables, n, _ = f.tables()
+    q = to_dev(rand_bits(rng, (1, H * R, T, D), dt), dt)
+    got = pool.attention(0, q, tables, n, T, 1.0 / np.sqrt(D)).cpu()
+    for end in (64, 2000, T):
+        m = i32([end])
+        want = pool.attention(0, q[:, :, end - 2:end].contiguous(), tables, m, T, 1.0 / np.sqrt(D)).cpu()  # 6 rows: VALU kernel
+        assert (got[:, :, end - 2:end] - want).abs().max() <= 2e-4  # two kernels, each within 1e-4 of fp64
+    pool.close()
+
+
+@pytest.mark.parametrize("mode", ["affine_g64", "ref_row"])
+@pytest.mark.parametrize("scale", [0.0, -0.05, 1.0])
+def test_scales(mode, scale):
+    print(f"\ncase long_window_scale mode={mode} scale={scale}", flush=True)
+    got, ref = _run(mode, 128, 1, 4, [150, 400], 20, scale=scale, seed=11)
+    assert np.abs(got - ref).max() <= ATOL
+
+
+@pytest.mark.parametrize("mode", ["affine_g64", "ref_row"])
+def test_queries_beyond_fp16(mode):
+    """bf16 queries past fp16's range: scaled by 2^-k, their scores by 2^k."""
+    print(f"\ncase long_window_qrange mode={mode}", flush=True)
+    got, ref = _run(mode, 64, 1, 4, [130, 200], 18, scale=2.0 ** -18, q_mul=1e6, seed=13)
+    assert np.abs(got - ref).max() <= ATOL
+
+
+@pytest.mark.parametrize("D", [128, 512])
+@pytest.mark.parametrize("out", [torch.bfloat16, torch.float16])
+def test_low_precision_output(D, out):
+    print(f"\ncase long_window_out D={D} {out}", flush=True)
+    got, ref = _run("affine_g64", D, 1, 4, [40, 333], 19, out_dtype=out, split_blocks=2, seed=17)
+    ulp = 2.0 ** -8 if out is torch.bfloat16 else 2.0 ** -11
+    assert (np.abs(got - ref) - ulp * np.abs(ref)).max() <= ATOL
+
+
+def test_many_query_heads_per_kv_head():
+    """One new row, 70 query heads per KV head: the same kernel, decode's plan."""
+    print("\ncase long_window_mqa", flush=True)
+    got, ref = _run("affine_g64", 64, 1, 70, [1, 64, 500], 1, seed=19)
+    assert np.abs(got - ref).max() <= ATOL
+
+
+@pytest.mark.parametrize("mode", ["affine_g64", "ref_row"])
+def test_batch_past_one_wave_of_lengths(mode):
+    """70 sequences: lengths past the 64 a wave holds in one register."""
+    print(f"\ncase long_window_batch mode={mode}", flush=True)
+    rng = np.random.default_rng(23)
+    lens = [int(x) for x in rng.integers(33, 200, size=70)]
+    got, ref = _run(mode, 64, 1, 2, lens, 33, seed=29)
+    assert np.abs(got - ref).max() <= ATOL
