@@ -1327,9 +1327,38 @@ hipError_t launch_attention_windowed(const PoolGeometry &g, int32_t layer, const
   return launch_attention(g, layer, w, p, st);
 }
 
+// Short sequences on the decode kernel: a workgroup per (sequence, KV head)
+// whose waves combine their partials in LDS (the window variants, with a
+// window that hides nothing) saves the merge launch, and while a wave has at
+// most about 1.5 blocks it costs no time to leave the flat split's other
+// waves idle.  Measured per fused RoPE call, batches of 1 / 32, flat split
+// against this: head_dim 64, 256 tokens 13.6 / 16.5 against 11.5 / 12.3 us;
+// head_dim 128, 5 rows, 512 tokens 20.4 / 25.8 against 18.1 / 21.2; head_dim
+// 256, 512 tokens 21.8 / 32.7 against 18.7 / 25.2.  At 2 to 2.5 blocks a wave
+// the two meet (128 dims, 5 rows, 1024 tokens, batch of 4: 22.0 against 22.4;
+// 8 rows, whose LDS leaves 4 waves: 24.2 against 22.9 at 512, 24.7 against
+// 28.8 at 1024), and with ragged lengths the longest sequence decides.  One
+// workgroup fills a compute unit: past one round of them (384 workgroups on
+// 256 units, 128 dims, lengths 10-320) the flat split is faster, 24.2 against
+// 31.2 us.
+static bool per_sequence_decode(const PoolGeometry &g, const AttnLaunch &a, const AttnPlan &p) {
+  if (p.use_mfma || g.D > 256 || p.split_blocks > 0) return false;
+  if (a.window > 0 || a.partial_only || a.len_const >= 0 || !a.causal) return false;
+  if (a.rope_cs && (!a.k_new || a.Lq != 1)) return false;
+  if ((int64_t)a.B * g.Hkv > g.num_cus) return false;
+  const int32_t waves = valu_window_limit(g, p.NR, a.rope_cs != nullptr) / (64 * 64);
+  return 2 * p.nb_cap <= 3 * waves;
+}
+
 hipError_t launch_attention(const PoolGeometry &g, int32_t layer, const AttnLaunch &a, const AttnPlan &p,
                             hipStream_t st) {
   if (a.B == 0) return hipSuccess;
+  if (per_sequence_decode(g, a, p)) {
+    AttnLaunch w = a;
+    w.win_start = nullptr;
+    w.window = 1 << 30;
+    return launch_attn_valu(g, layer, w, p, st);
+  }
   if (a.k_new && p.use_mfma) {
     hipError_t e = launch_append_newest(g, layer, a, p, st);
     if (e != hipSuccess) return e;
