@@ -74,6 +74,11 @@ __device__ __forceinline__ half2_t rest_pair(float w0, float w1, half2_t h, floa
 // core for four VALU slots, and a wave issues in order, so products and VALU
 // work only overlap within a wave where they alternate).
 __device__ __forceinline__ void fence_all() { __builtin_amdgcn_sched_barrier(0); }
+// A raised reference lies this far below the row's maximum (log2 units): the
+// weights then sit high in fp16's range, where the low parts of p s_v keep
+// their 11 bits (at the maximum itself most were subnormal: 4.8e-6 of the
+// result against 64 bits, about 2e-7 so), under the same bound of 2^8.
+constexpr float kMaxGap = 5.0f;
 // No LDS read crosses: what is read above stays above, in flight.
 __device__ __forceinline__ void fence_lds() { __builtin_amdgcn_sched_barrier(0x47f); }
 
@@ -536,14 +541,16 @@ __global__ __launch_bounds__(256, (prefill_min_waves<D, NRT>())) void k_attn_pre
           }
         } else {
           fence_lds();
-          if (c == 0) {
+          // (a chain of 128 dims, then one sum: head_dim 512 in one chain of
+          // 16 products rounds worse, 2.6e-7 against 1.7e-7)
 #pragma unroll
-            for (int rt = 0; rt < NRT; ++rt) sc[t][rt] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+          for (int rt = 0; rt < NRT; ++rt) {
+            float4_t v = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            if (CPT <= 2 && c > 0) v = sc[t][rt];
+#pragma unroll
+            for (int j = 0; j < CH; ++j) v = mfma16x16x32(fr[u & 1][j], qB[rt][CH * c + j], v);
+            sc[t][rt] = CPT <= 2 || c == 0 ? v : sc[t][rt] + v;
           }
-#pragma unroll
-          for (int j = 0; j < CH; ++j)
-#pragma unroll
-            for (int rt = 0; rt < NRT; ++rt) sc[t][rt] = mfma16x16x32(fr[u & 1][j], qB[rt][CH * c + j], sc[t][rt]);
         }
       }
       if constexpr (AFF) {
@@ -576,10 +583,10 @@ __global__ __launch_bounds__(256, (prefill_min_waves<D, NRT>())) void k_attn_pre
             }
       }
 
-      // ---- online softmax with a lazily raised running max (log2 units; the
-      // row's 64 scores live in lanes n, n+16, n+32, n+48): it only moves
-      // when some score exceeds it by more than 8, so the weights stay below
-      // 2^8 and most blocks skip the rescale
+      // ---- online softmax with a lazily raised running reference m (log2
+      // units; the row's 64 scores live in lanes n, n+16, n+32, n+48): it
+      // only moves when some score exceeds it by more than 8, so the weights
+      // stay below 2^8 and most blocks skip the rescale
       // (affine mode: scores relative to the running max, 0 before the first)
       float mb[NRT];
       bool over = false;
@@ -605,7 +612,7 @@ __global__ __launch_bounds__(256, (prefill_min_waves<D, NRT>())) void k_attn_pre
 #pragma unroll
         for (int rt = 0; rt < NRT; ++rt) {
           const float mu = m_run[rt] == -INFINITY ? 0.0f : m_run[rt];
-          const float mn = fmaxf(m_run[rt], AFF ? mb[rt] + mu : mb[rt]);
+          const float mn = fmaxf(m_run[rt], (AFF ? mb[rt] + mu : mb[rt]) - kMaxGap);
           const float al = m_run[rt] == -INFINITY ? 0.0f : fast_exp2(m_run[rt] - mn);
           if constexpr (AFF) {
             const float down = mn == -INFINITY ? 0.0f : mn - mu;
