@@ -1251,7 +1251,9 @@ hipError_t launch_attn_merge(const PoolGeometry &g, int32_t layer, const AttnLau
                              hipStream_t st) {
   if (a.B == 0) return hipSuccess;
   const AttnArgs args = make_attn_args(g, layer, a, p);
-  if (p.prefill) {
+  // (few rows: one wave each, side by side -- 2 x 48 new rows, 3072 waves: the
+  // call takes 1 us less so; from 8192 on the workgroups are what costs)
+  if (p.prefill && (int64_t)p.NR * g.Hkv * a.B >= 8192) {
     const dim3 rows((unsigned)p.row_groups, (unsigned)g.Hkv, (unsigned)a.B);
     KRILL_DISPATCH_D(g.D, { k_attn_merge_rows<D><<<rows, dim3(256), 0, st>>>(args); });
     return hipGetLastError();
