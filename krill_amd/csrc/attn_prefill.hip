@@ -5,12 +5,12 @@
 // Sources/KrillEngine/BatchedDecode.swift:299-312), same flat block split,
 // same partial slots.
 //
-// Bound: the matrix cores and the VALU together.  Per (64 keys x 16 rows) the
-// matrix cores run D / 32 steps of Q.K^T and, the weights being pairs of fp16
-// operands, D / 16 of P.V; the VALU runs the softmax and the scales.  So the
-// work that does not depend on the rows is done once per workgroup (64 W / 4
-// to 128 rows), and what depends on (row, key) is kept to the fewest
-// instructions:
+// Bound: the matrix cores and the VALU in turn, and the clock, which falls to
+// 1.6 - 2.0 GHz under this load.  Per (64 keys x 16 rows) the matrix cores run
+// D / 32 steps of Q.K^T and, the weights being pairs of fp16 operands, twice
+// that of P.V; the VALU runs the softmax and the scales.  So the work that does
+// not depend on the rows is done once per workgroup of 64 or 128 rows, and what
+// depends on (row, key) is kept to the fewest instructions:
 //  * a block's K and V bytes go global -> registers -> fp16 tiles in LDS
 //    (exact u - 128; row mode: dequantized as the reference does), converted
 //    once for all waves; the next block's bytes are in flight meanwhile.
@@ -19,9 +19,15 @@
 //  * the zero-point term sum_g (z + 128 s)_g * (sum of q over group g) is a
 //    contraction over the scale groups: fp32 MFMA, four groups a step;
 //  * the softmax scale rides on the scales of K and the scores' accumulators
-//    start at minus the running maximum (row mode: both in the exponent's fma);
-//  * weights p * s_v are split into fp16 high and low parts by two mixed fmas
-//    each: hi = f16(p s), lo = f16(p s - hi).
+//    start at minus the running reference (row mode: both in the exponent's
+//    fma);
+//  * weights p * s_v are split into fp16 high and low parts in three full-rate
+//    instructions each, alternating with the products of the step before.
+// Measured, calls with their append (the verify kernel, or at head_dim 512 the
+// decode kernel, before): 8 x 512 rows on contexts of 2048-6144, Hq 40, D 128:
+// 753 us = 485 TFLOP/s (1073); a 3900-row prompt, row mode, Hq 32: 240 us = 520
+// TFLOP/s (533); 2 x 256 rows at head_dim 512: 134 us (288); 4 x 512 rows,
+// window 1024, head_dim 256: 162 us (298).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -41,8 +47,8 @@ struct PrefillLds {
   static constexpr bool AFF = MODE == MODE_AFFINE;
   __attribute__((aligned(16))) uint8_t k[64 * KTS];
   __attribute__((aligned(16))) uint8_t v[D * VTS];
-  __attribute__((aligned(16))) float ks[AFF ? G * 64 : 4];      // [g][token]
-  __attribute__((aligned(16))) float kz[AFF ? GZ * 64 : 4];     // [g][token]: z + 128 s
+  __attribute__((aligned(16))) float ks[AFF ? G * 64 : 4];      // [g][token]: s times the softmax scale
+  __attribute__((aligned(16))) float kz[AFF ? GZ * 64 : 4];     // [g][token]: z + 128 s, the same
   __attribute__((aligned(16))) float vz[AFF ? G * 64 : 4];      // [g][position]: z + 128 s
   __attribute__((aligned(16))) _Float16 vs[AFF ? G * 64 : 8];   // [g][position]
 };
