@@ -90,6 +90,38 @@ __device__ __forceinline__ void fence_lds() { __builtin_amdgcn_sched_barrier(0x4
 
 // Waves of a workgroup: one per (32-token group, 16-position half) of a V row.
 constexpr int kPrefillWaves = 4;
+// Where in a head region the loads of a block lie: piece k of wave `wid` starts
+// at `piece` bytes (a scalar offset), each lane reads at its own offset from
+// there.  The range check of a buffer load does not cover the scalar offset, so
+// the sums must lie in the region by themselves.
+constexpr int prefill_k_piece(int wid, int k) { return (wid + kPrefillWaves * k) * 1024; }
+template <int D>
+constexpr int prefill_v_piece(int wid, int k) {
+  return v_offset(D) + ((wid >> 1) & 1) * 32 * D + (wid & 1) * 1024 + k * (64 / (D / 64) * 16);
+}
+// row `lane` of a 64-row run of V^T
+template <int D>
+constexpr int prefill_v_lane(int lane) { return 2 * (lane % (D / 64)) * 1024 + lane / (D / 64) * 16; }
+// affine metadata, runs of 64 words: 128 G words, at G = 1 half of what the four
+// waves would load -- the other two read the same words again (unused)
+template <int D, int G>
+constexpr int prefill_meta_piece(int wid, int k) {
+  const int run = wid + kPrefillWaves * k;
+  return km_offset(D) + 256 * (2 * G < kPrefillWaves ? run % (2 * G) : run);
+}
+template <int D, int G>
+constexpr bool prefill_loads_inside(int k_pieces, int v_pieces, int meta_pieces) {
+  for (int w = 0; w < kPrefillWaves; ++w)
+    for (int lane = 0; lane < 64; ++lane) {
+      for (int k = 0; k < k_pieces; ++k)
+        if (prefill_k_piece(w, k) + 16 * lane + 16 > v_offset(D)) return false;
+      for (int k = 0; k < v_pieces; ++k)
+        if (prefill_v_piece<D>(w, k) + prefill_v_lane<D>(lane) + 16 > km_offset(D)) return false;
+      for (int k = 0; k < meta_pieces; ++k)
+        if (prefill_meta_piece<D, G>(w, k) + 4 * lane + 4 > head_region_bytes(D, G)) return false;
+    }
+  return true;
+}
 // Waves per SIMD the registers are budgeted for: the accumulators and queries
 // of NRT row tiles take 6 NRT D / 16 registers a lane.
 template <int D, int NRT>
@@ -109,6 +141,7 @@ __global__ __launch_bounds__(256, (prefill_min_waves<D, NRT>())) void k_attn_pre
   constexpr int VP = D / 16 / W;  // 16-byte V pieces per thread
   constexpr int MW = AFF ? (128 * G + 64 * W - 1) / (64 * W) : 0;  // metadata words per thread
   static_assert(W == 4 && D % 64 == 0, "a wave per (token group, half) of V");
+  static_assert(prefill_loads_inside<D, G>(KP, VP, MW), "a block's loads stay in its head region");
   using Lds = PrefillLds<D, MODE>;
   constexpr int KTS = Lds::KTS, VTS = Lds::VTS;
   __shared__ Lds lds;
@@ -189,10 +222,10 @@ __global__ __launch_bounds__(256, (prefill_min_waves<D, NRT>())) void k_attn_pre
   uint4 kraw[KP], vraw[VP];
   uint32_t mraw[AFF ? MW : 1];  // affine: words tid + 64 W k of the block's metadata; row mode: K word of token `lane`
   uint32_t vmeta = 0u;          // row mode: V word of token `lane`
-  constexpr int DPL = D / 64;
-  const int vlane = 2 * (lane % DPL) * 1024 + lane / DPL * 16;  // row `lane` of a 64-row run of V^T
+  const int vlane = prefill_v_lane<D>(lane);
   auto issue = [&](int i) {
-    // after the last block: an empty resource, no memory access
+    // after the last block: an empty resource (the offsets in scalars may escape
+    // the range check: then block 0 or a block of this range is read, unused)
     const int bytes = __builtin_amdgcn_readfirstlane(i < iend ? a.lv.head_bytes : 0);
     if (i < iend && i - tab0 == 64) load_table(i);
     const int phys = __builtin_amdgcn_readlane(tab, __builtin_amdgcn_readfirstlane((i - tab0) & 63));
@@ -202,14 +235,13 @@ __global__ __launch_bounds__(256, (prefill_min_waves<D, NRT>())) void k_attn_pre
       return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 0));
     };
 #pragma unroll
-    for (int k = 0; k < KP; ++k) kraw[k] = ld16(lane * 16, (wid + W * k) * 1024);
+    for (int k = 0; k < KP; ++k) kraw[k] = ld16(lane * 16, prefill_k_piece(wid, k));
 #pragma unroll
-    for (int k = 0; k < VP; ++k)
-      vraw[k] = ld16(vlane, v_offset(D) + vtg * 32 * D + vh * 1024 + k * (64 / DPL * 16));
+    for (int k = 0; k < VP; ++k) vraw[k] = ld16(vlane, prefill_v_piece<D>(wid, k));
     if constexpr (AFF) {
 #pragma unroll
       for (int k = 0; k < MW; ++k)
-        mraw[k] = __builtin_amdgcn_raw_buffer_load_b32(r, lane * 4, km_offset(D) + (64 * wid + 64 * W * k) * 4, 0);
+        mraw[k] = __builtin_amdgcn_raw_buffer_load_b32(r, lane * 4, prefill_meta_piece<D, G>(wid, k), 0);
     } else {
       mraw[0] = __builtin_amdgcn_raw_buffer_load_b32(r, lane * 4, km_offset(D), 0);
       vmeta = __builtin_amdgcn_raw_buffer_load_b32(r, lane * 4, vm_offset(D, G), 0);

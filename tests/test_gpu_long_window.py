@@ -116,3 +116,22 @@ def test_batch_past_one_wave_of_lengths(mode):
     lens = [int(x) for x in rng.integers(33, 200, size=70)]
     got, ref = _run(mode, 64, 1, 2, lens, 33, seed=29)
     assert np.abs(got - ref).max() <= ATOL
+
+
+def test_blocks_at_the_pools_end():
+    """head_dim 64, affine: 128 metadata words a block for 256 threads, in a pool whose last
+    layer's last block is attended (that no load leaves a block's region is asserted where the
+    kernel is compiled)."""
+    print("\ncase long_window_pool_end", flush=True)
+    rng = np.random.default_rng(31)
+    lens, H, R, D, Lq = [128, 200, 64], 2, 4, 64, 20
+    pool = krill_amd.KVPool(2, H, D, sum((n + 63) // 64 for n in lens), "affine_g64", "bf16", free_list_seed=1)
+    f = Filled(pool, lens, rng, "bf16", layers=(1,))
+    tables, n, _ = f.tables()
+    assert int(tables.max()) == pool.num_blocks - 1
+    q = rand_bits(rng, (len(lens), H * R, Lq, D), "bf16")
+    got = pool.attention(1, to_dev(q, "bf16"), tables, n, max(lens), 0.125)
+    torch.cuda.synchronize()
+    ref = oracle_attention(pool, f, 1, q, "bf16", 0.125)
+    pool.close()
+    assert np.abs(got.double().cpu().numpy() - ref).max() <= ATOL
