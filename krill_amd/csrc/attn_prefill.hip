@@ -25,7 +25,7 @@
 //    instructions each, alternating with the products of the step before.
 // Measured, calls with their append (the verify kernel, or at head_dim 512 the
 // decode kernel, before): 8 x 512 rows on contexts of 2048-6144, Hq 40, D 128:
-// 753 us = 485 TFLOP/s (1073); a 3900-row prompt, row mode, Hq 32: 240 us = 520
+// 762 us = 479 TFLOP/s (1073); a 3900-row prompt, row mode, Hq 32: 240 us = 520
 // TFLOP/s (533); 2 x 256 rows at head_dim 512: 134 us (288); 4 x 512 rows,
 // window 1024, head_dim 256: 162 us (298).
 #include <hip/hip_runtime.h>
@@ -51,6 +51,7 @@ struct PrefillLds {
   __attribute__((aligned(16))) float kz[AFF ? GZ * 64 : 4];     // [g][token]: z + 128 s, the same
   __attribute__((aligned(16))) float vz[AFF ? G * 64 : 4];      // [g][position]: z + 128 s
   __attribute__((aligned(16))) _Float16 vs[AFF ? G * 64 : 8];   // [g][position]
+  int big;  // last block with a V scale past kBigScale
 };
 
 __device__ __forceinline__ float4_t mfma16x16x4f32(float a, float b, float4_t c) {
@@ -80,11 +81,16 @@ __device__ __forceinline__ half2_t rest_pair(float w0, float w1, half2_t h, floa
 // core for four VALU slots, and a wave issues in order, so products and VALU
 // work only overlap within a wave where they alternate).
 __device__ __forceinline__ void fence_all() { __builtin_amdgcn_sched_barrier(0); }
-// A raised reference lies this far below the row's maximum (log2 units): the
+// A raised reference lies kMaxGap below the row's maximum (log2 units): the
 // weights then sit high in fp16's range, where the low parts of p s_v keep
 // their 11 bits (at the maximum itself most were subnormal: 4.8e-6 of the
-// result against 64 bits, about 2e-7 so), under the same bound of 2^8.
-constexpr float kMaxGap = 5.0f;
+// result against 64 bits, about 2e-7 so).  It is raised when a score exceeds it
+// by kMaxOver, so p < 2^8 and p s_v stays finite in fp16 for |s_v| <= kBigScale
+// (V values of some +-32000 in one group, or scales brought in from outside).
+// A block with a larger scale raises it to the maximum itself: p <= 1 there.
+// (The test takes 9 of 762 us on the 8 x 512-row chunks; kMaxOver 6.9, which
+// bounds p s_v for the quantizer's own scales only, takes the same: more raises.)
+constexpr float kMaxGap = 5.0f, kMaxOver = 8.0f, kBigScale = 248.0f;
 // No LDS read crosses: what is read above stays above, in flight.
 __device__ __forceinline__ void fence_lds() { __builtin_amdgcn_sched_barrier(0x47f); }
 
@@ -389,6 +395,7 @@ __global__ __launch_bounds__(256, (prefill_min_waves<D, NRT>())) void k_attn_pre
   if constexpr (AFF && Lds::GZ > G) {  // the zero-point contraction's unused groups
     for (int k = tid; k < (Lds::GZ - G) * 64; k += 64 * W) lds.kz[G * 64 + k] = 0.0f;
   }
+  if (AFF && tid == 0) lds.big = -1;
   issue(i0);
   load_q(b);
 
@@ -469,6 +476,7 @@ __global__ __launch_bounds__(256, (prefill_min_waves<D, NRT>())) void k_attn_pre
             const int p = (t & 32) + vpos(t & 31);
             lds.vs[g * 64 + p] = data ? sh : (_Float16)0.0f;
             lds.vz[g * 64 + p] = data ? zf : 0.0f;
+            if (data && fabsf(sf) > kBigScale) lds.big = i;
           }
         }
       } else {
@@ -591,7 +599,9 @@ __global__ __launch_bounds__(256, (prefill_min_waves<D, NRT>())) void k_attn_pre
           }
         }
       }
+      float over_by = kMaxOver;
       if constexpr (AFF) {
+        if (lds.big == i) over_by = 0.0f;
 #pragma unroll
         for (int rt = 0; rt < NRT; ++rt) {
           scale(NGRP - 1, rt, 0);
@@ -623,8 +633,8 @@ __global__ __launch_bounds__(256, (prefill_min_waves<D, NRT>())) void k_attn_pre
 
       // ---- online softmax with a lazily raised running reference m (log2
       // units; the row's 64 scores live in lanes n, n+16, n+32, n+48): it
-      // only moves when some score exceeds it by more than 8, so the weights
-      // stay below 2^8 and most blocks skip the rescale
+      // only moves when some score exceeds it by more than kMaxOver, so the
+      // weights stay below 2^8 and most blocks skip the rescale
       // (affine mode: scores relative to the running max, 0 before the first)
       float mb[NRT];
       bool over = false;
@@ -640,24 +650,25 @@ __global__ __launch_bounds__(256, (prefill_min_waves<D, NRT>())) void k_attn_pre
         v = max2(va, vb);
         if constexpr (AFF) {
           mb[rt] = v;
-          over |= v > (m_run[rt] == -INFINITY ? -INFINITY : 8.0f);
+          over |= v > (m_run[rt] == -INFINITY ? -INFINITY : over_by);
         } else {
           mb[rt] = v * q_up[AFF ? 0 : rt];
-          over |= mb[rt] > m_run[rt] + 8.0f;
+          over |= mb[rt] > m_run[rt] + over_by;
         }
       }
       if (__any(over)) {
+        const float gap = AFF && over_by == 0.0f ? 0.0f : kMaxGap;
 #pragma unroll
         for (int rt = 0; rt < NRT; ++rt) {
           const float mu = m_run[rt] == -INFINITY ? 0.0f : m_run[rt];
-          const float mn = fmaxf(m_run[rt], (AFF ? mb[rt] + mu : mb[rt]) - kMaxGap);
+          const float mn = fmaxf(m_run[rt], (AFF ? mb[rt] + mu : mb[rt]) - gap);
           const float al = m_run[rt] == -INFINITY ? 0.0f : fast_exp2(m_run[rt] - mn);
           if constexpr (AFF) {
             const float down = mn == -INFINITY ? 0.0f : mn - mu;
 #pragma unroll
             for (int t = 0; t < 4; ++t)
 #pragma unroll
-              for (int x = 0; x < 4; ++x) sc[t][rt][x] -= down;
+              for (int x = 0; x < 4; ++x) sc[t][rt][x] = fminf(sc[t][rt][x] - down, gap);
             nm[rt] = mn == -INFINITY ? 0.0f : -mn * q_dn[rt];
           }
           m_run[rt] = mn;
