@@ -1223,11 +1223,12 @@ int32_t plan_attention(const PoolGeometry &g, int32_t B, int32_t Hq, int32_t Lq,
     waves = (tmax + pw - 1) / pw;
   } else if (p.use_mfma) {
     const int64_t groups = (p.row_groups + p.group_waves - 1) / p.group_waves;
-    const int64_t per_cu = p.prefill ? prefill_groups_per_cu(g)
-                                     : mfma_groups_per_cu(g, p.group_waves, p.token_split);
+    int64_t per_cu = p.prefill ? prefill_groups_per_cu(g) : mfma_groups_per_cu(g, p.group_waves, p.token_split);
+    // (a decode step takes no more ranges than the verify kernel's groups of
+    // four would, so its workspace stays within the static scratch it had)
+    if (p.prefill && Lq == 1) per_cu = std::min<int64_t>(per_cu, mfma_groups_per_cu(g, 4, 1));
     const int64_t cap = cus * per_cu, hg = (int64_t)g.Hkv * groups;
     waves = std::max<int64_t>(1, cap / hg);
-    // (a decode step's workspace stays within the static scratch it had)
     if (p.prefill && Lq > 1) waves = prefill_ranges(cap, hg);
   } else if (dsplit) {
     // workgroups of 4 waves (one per 128-dim slice)

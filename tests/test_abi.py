@@ -62,6 +62,15 @@ def test_kernels_refuse_host_only_pools():
     assert lib.krill_copy_blocks(p.handle, dummy, 1, None) == L.KRILL_E_STATE
 
 
+@pytest.mark.parametrize("B", [1, 8, 15])
+def test_one_row_step_of_many_query_heads_fits_the_static_scratch(B):
+    """head_dim 256, affine, 65 to 128 query heads per KV head, one new row: the allocation-free
+    step's 32 MiB hold its partials (8 row groups of 16, 128 ranges at most)."""
+    p = krill_amd.KVPool(1, 1, 256, 64, "affine_g64", host_only=True)
+    for Hq in range(65, 129):
+        assert p.workspace_size(B, Hq, 1, 4096) <= 32 << 20, Hq
+
+
 def test_workspace_size_and_path_limits():
     p = krill_amd.KVPool(1, 8, 128, 64, host_only=True)
     ws = p.workspace_size(32, 40, 1, 8192)

@@ -101,6 +101,19 @@ def test_noalloc_step_matches_the_workspace_entry_point(mode):
         p.close()
 
 
+def test_noalloc_step_of_many_query_heads():
+    """128 query heads on one KV head of 256 dims: the step runs in the static scratch."""
+    print("\ncase noalloc many heads", flush=True)
+    dt, R, D, prefill = "bf16", 128, 256, [300, 64, 1025]
+    pools = [krill_amd.KVPool(1, 1, D, 32, "affine_g64", dt, free_list_seed=7) for _ in range(2)]
+    fills = [Filled(p, prefill, np.random.default_rng(81), dt) for p in pools]
+    out_ws, out_na, tables, full = _step(pools, fills, [0, 1, 2], np.random.default_rng(82), dt, R)
+    assert torch.equal(out_ws, out_na)
+    _same_pool_bytes(pools, tables, full)
+    for p in pools:
+        p.close()
+
+
 def test_noalloc_refuses_a_step_beyond_the_scratch():
     """Short sequences in a batch large enough that the step's workspace
     exceeds the scratch: KRILL_E_RANGE before any launch, the output left as
