@@ -1120,23 +1120,26 @@ hipError_t launch_copy_pairs(const PoolGeometry &g, const CopyPair *pairs, int32
   return hipSuccess;
 }
 
-// Block ranges per (KV head, row-group workgroup) of the long-window kernel,
-// hg such workgroups on a chip that holds `cap`: the first k (rounds of
-// resident workgroups) whose floor(k cap / hg) ranges fill at least 90 % of
-// them, else the fullest of the first eight.
-static int64_t prefill_ranges(int64_t cap, int64_t hg) {
-  int64_t best = 1;
-  double fill = 0.0;
-  const int64_t k0 = (hg + cap - 1) / cap;
-  for (int64_t k = k0; k < k0 + 8 && fill < 0.9; ++k) {
+// Block ranges per (KV head, row-group workgroup) of the long-window kernel: hg
+// such workgroups on a chip that holds `cap`, tmax blocks at most each.  One
+// round of resident workgroups, unless that leaves a quarter of the chip idle
+// and the ranges of some further rounds fill 85 % of it with 10 blocks or more
+// each: every round costs its workgroups' start and epilogue, some 5 blocks'
+// time, and every range its partials.  Measured, one round against this rule:
+// Hq 40, D 128, 1000 rows on 4000 tokens (79 blocks, 320 of 512 workgroups) 280
+// against 215 us; D 256, 700 rows on 4000 (352 of 512) 180 against 158.  Below
+// 10 blocks a range more rounds lose: Hq 40, 2 x 512 rows on 300 tokens (8.7
+// blocks) 67 against 72 us, 700 rows on 300 (2 blocks) 45 against 92; and where
+// one round fills 89 %, 6 x 300 rows on 1000 tokens, 92 against 130.
+static int64_t prefill_ranges(int64_t cap, int64_t hg, int64_t tmax) {
+  const int64_t one = std::max<int64_t>(1, cap / hg), k0 = (hg + cap - 1) / cap;
+  if (4 * one * hg >= 3 * k0 * cap) return one;
+  for (int64_t k = k0 + 1; k <= k0 + 7; ++k) {
     const int64_t w = k * cap / hg;
-    const double f = (double)(w * hg) / (double)(k * cap);
-    if (f > fill + 1e-9) {
-      fill = f;
-      best = w;
-    }
+    if (tmax < 10 * w) break;
+    if (20 * w * hg >= 17 * k * cap) return w;
   }
-  return best;
+  return one;
 }
 
 int32_t plan_attention(const PoolGeometry &g, int32_t B, int32_t Hq, int32_t Lq, int32_t max_seq_len,
@@ -1228,8 +1231,7 @@ int32_t plan_attention(const PoolGeometry &g, int32_t B, int32_t Hq, int32_t Lq,
     // four would, so its workspace stays within the static scratch it had)
     if (p.prefill && Lq == 1) per_cu = std::min<int64_t>(per_cu, mfma_groups_per_cu(g, 4, 1));
     const int64_t cap = cus * per_cu, hg = (int64_t)g.Hkv * groups;
-    waves = std::max<int64_t>(1, cap / hg);
-    if (p.prefill && Lq > 1) waves = prefill_ranges(cap, hg);
+    waves = p.prefill && Lq > 1 ? prefill_ranges(cap, hg, tmax) : std::max<int64_t>(1, cap / hg);
   } else if (dsplit) {
     // workgroups of 4 waves (one per 128-dim slice)
     const int64_t wg_per_cu = std::max<int32_t>(1, valu_waves_per_cu(g, p.rows_per_group) / (g.D / 128));

@@ -71,6 +71,21 @@ def test_one_row_step_of_many_query_heads_fits_the_static_scratch(B):
         assert p.workspace_size(B, Hq, 1, 4096) <= 32 << 20, Hq
 
 
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_long_window_workspace_holds_one_round_of_ranges(D):
+    """Chunks of 200 to 1000 rows on 0 to 500 tokens of one sequence: no more block ranges than
+    one round of resident workgroups (two per compute unit, 256 of those) takes.  More rounds
+    only pay where each range keeps 10 blocks."""
+    for H, R in ((8, 4), (8, 5), (4, 8), (8, 2)):
+        p = krill_amd.KVPool(1, H, D, 64, host_only=True)
+        for Lq in range(200, 1001, 50):
+            for T in (0, 100, 300, 500):
+                rows = 64 * ((R * Lq + 63) // 64)  # the row groups of 16 or 32, to whole workgroups
+                ranges = max(1, 512 // (H * (rows // 128)))
+                bound = H * (rows + 64) * (ranges + 1) * (D + 2) * 4 + 512
+                assert p.workspace_size(1, H * R, Lq, Lq + T) <= bound, (H, R, Lq, T)
+
+
 def test_workspace_size_and_path_limits():
     p = krill_amd.KVPool(1, 8, 128, 64, host_only=True)
     ws = p.workspace_size(32, 40, 1, 8192)

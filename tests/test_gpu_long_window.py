@@ -56,25 +56,50 @@ def test_ranges_across_sequences(mode, D, split):
     assert np.abs(got - ref).max() <= ATOL
 
 
-@pytest.mark.parametrize("mode", ["affine_g64", "ref_row"])
-def test_range_longer_than_the_table_window(mode):
-    """A whole prompt of 72 blocks on 8 KV heads, 108 row-group workgroups each, so many that each
-    takes its rows' whole range: up to 72 blocks, past the 64 table entries a workgroup holds at
-    once.  Checked on rows of the first, a middle and the last blocks against the same rows as a
-    short window."""
-    print(f"\ncase long_window_table mode={mode}", flush=True)
-    H, R, D, T, dt = 8, 3, 128, 72 * 64 - 5, "bf16"
-    rng = np.random.default_rng(3)
-    pool = krill_amd.KVPool(1, H, D, 80, mode, dt, free_list_seed=9)
-    f = Filled(pool, [T], rng, dt, max_chunk=4000)
+def _ranges(pool, B, Hq, Lq, mx, tile):
+    """Block ranges per row group, from the workspace: a slot per (KV head, row group) and range
+    or sequence, `tile` rows of D values and two more each."""
+    groups = (Hq // pool.num_kv_heads * Lq + tile - 1) // tile
+    slots = pool.workspace_size(B, Hq, Lq, mx) // (tile * (pool.head_dim + 2) * 4)
+    return slots // (pool.num_kv_heads * groups) - B
+
+
+def _rows_against_short_windows(pool, lens, Lq, R, seed, at, ranges, tile=32):
+    """Rows `at` (offsets into the new rows) of a long window against the same rows as windows of
+    two, which run on the decode kernel (two kernels, each within 1e-4 of fp64)."""
+    rng = np.random.default_rng(seed)
+    H, D, dt = pool.num_kv_heads, pool.head_dim, "bf16"
+    f = Filled(pool, lens, rng, dt, max_chunk=4000)
     tables, n, _ = f.tables()
-    q = to_dev(rand_bits(rng, (1, H * R, T, D), dt), dt)
-    got = pool.attention(0, q, tables, n, T, 1.0 / np.sqrt(D)).cpu()
-    for end in (64, 2000, T):
-        m = i32([end])
-        want = pool.attention(0, q[:, :, end - 2:end].contiguous(), tables, m, T, 1.0 / np.sqrt(D)).cpu()  # 6 rows: VALU kernel
-        assert (got[:, :, end - 2:end] - want).abs().max() <= 2e-4  # two kernels, each within 1e-4 of fp64
+    assert _ranges(pool, len(lens), H * R, Lq, max(lens), tile) == ranges
+    q = to_dev(rand_bits(rng, (len(lens), H * R, Lq, D), dt), dt)
+    got = pool.attention(0, q, tables, n, max(lens), 1.0 / np.sqrt(D)).cpu()
+    for j in at:
+        m = i32([T - Lq + j for T in lens])
+        want = pool.attention(0, q[:, :, j - 2:j].contiguous(), tables, m, max(lens), 1.0 / np.sqrt(D)).cpu()
+        assert (got[:, :, j - 2:j] - want).abs().max() <= 2e-4
     pool.close()
+
+
+@pytest.mark.parametrize("mode", ["affine_g64", "ref_row"])
+@pytest.mark.parametrize("lens,Lq,R", [([72 * 64 - 5], 72 * 64 - 5, 3), ([50 * 64 - 9, 36 * 64], 2048, 4)])
+def test_range_longer_than_the_table_window(mode, lens, Lq, R):
+    """So many row-group workgroups that each takes its rows' whole range, past the 64 table
+    entries a workgroup holds at once: a prompt of 72 blocks, and a second sequence whose blocks
+    51 to 86 of the range cross the 64th."""
+    print(f"\ncase long_window_table mode={mode} lens={lens}", flush=True)
+    pool = krill_amd.KVPool(1, 8, 128, sum((T + 63) // 64 for T in lens) + 4, mode, "bf16", free_list_seed=9)
+    _rows_against_short_windows(pool, lens, Lq, R, 3, (64, 1000, Lq), ranges=1)
+
+
+@pytest.mark.parametrize("mode", ["affine_g64", "ref_row"])
+@pytest.mark.parametrize("D,R,Lq,T,ranges,tile", [(128, 5, 1000, 5000, 3, 32), (256, 2, 700, 4700, 5, 16)])
+def test_more_rounds_of_ranges(mode, D, R, Lq, T, ranges, tile):
+    """Row groups that fill under three quarters of the chip over many blocks: two rounds of
+    ranges (one round: 1 and 2)."""
+    print(f"\ncase long_window_rounds mode={mode} D={D}", flush=True)
+    pool = krill_amd.KVPool(1, 8, D, (T + 63) // 64 + 4, mode, "bf16", free_list_seed=9)
+    _rows_against_short_windows(pool, [T], Lq, R, 5, (2, 500, Lq), ranges, tile)
 
 
 @pytest.mark.parametrize("mode", ["affine_g64", "ref_row"])
