@@ -1,6 +1,6 @@
 // Paged int8 attention with MFMA tiles: the speculative-verify path, used
-// when a KV head serves 9 to 64 query rows (GQA group x new tokens; longer
-// windows: attn_prefill.hip).  Reference semantics: the same SDPA call with
+// when a KV head serves 9 to 64 query rows (GQA group x new tokens), or more
+// over few blocks (other longer windows: attn_prefill.hip).  Reference semantics: the same SDPA call with
 // L > 1 new rows and the block-causal mask of
 // Sources/KrillEngine/BatchedDecode.swift:299-312 (row j of the new window
 // sees every cached key plus new keys 0..j), equivalently

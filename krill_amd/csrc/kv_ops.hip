@@ -1142,6 +1142,31 @@ static int64_t prefill_ranges(int64_t cap, int64_t hg, int64_t tmax) {
   return one;
 }
 
+// Whether the long-window kernel is the faster one for NR > 64 rows per KV head
+// over B sequences of at most nb blocks.  It converts each block for a whole
+// workgroup before any product, which pays from the second block of a range on:
+// while an even split leaves fewer, the kernel that starts sooner wins, the
+// verify kernel (the decode kernel at head_dim 512) -- unless one block is all a
+// sequence has, or at many rows.  The lines are from 2444 calls of 9 to 300 new
+// rows on 0 to 3000 tokens (plain, windowed, prefixes; one to eight sequences).
+// Either side of each, verify or decode kernel against this one, us of GPU time:
+//   head_dim 512  2 x 100 rows on 0 tokens 25.3 / 28.7; 1 x 200 on 1000 81 / 51;
+//                 2 x 130 on 0 (many rows) 44 / 31
+//   256, affine   1 x 100 on 300 22.3 / 26.2; 4 x 200 on 300 56.9 / 50.1
+//   256, row      1 x 100 on 100 19.8 / 21.8; 4 x 100 on 300 38.2 / 33.7
+//   128, affine   1 x 48 on 100 14.6 / 16.3; 1 x 48 on 0 14.5 / 13.0;
+//                 4 x 100 on 100 37.1 / 31.1 (Hq 40)
+//   128, row      1 x 17 on 100 13.3 / 13.7; 1 x 48 on 1000 25.8 / 23.7
+static bool long_window_faster(const PoolGeometry &g, int64_t B, int64_t nb, int64_t NR, int64_t cus) {
+  const int64_t groups = ((NR + 15) / 16 + 3) / 4, tmax = B * nb;
+  const int64_t ranges = std::max<int64_t>(1, cus * prefill_groups_per_cu(g) / (g.Hkv * groups));
+  const bool many = NR * g.Hkv * B > 4096;
+  if (g.D > 256) return tmax > ranges || (many && 4 * tmax > ranges);
+  if (g.D == 64 || nb == 1 || (g.D == 128 && many)) return true;
+  if (g.mode == MODE_REF) return 4 * tmax > ranges;
+  return 2 * tmax > (g.D == 256 ? 3 : 1) * ranges;
+}
+
 int32_t plan_attention(const PoolGeometry &g, int32_t B, int32_t Hq, int32_t Lq, int32_t max_seq_len,
                        int32_t split_blocks, int32_t path, AttnPlan *plan) {
   if (g.Hkv <= 0 || Hq <= 0 || Hq % g.Hkv != 0 || Lq <= 0 || B < 0 || max_seq_len < 0) return -1;
@@ -1154,15 +1179,17 @@ int32_t plan_attention(const PoolGeometry &g, int32_t B, int32_t Hq, int32_t Lq,
   // one grid row group each, every group reading all of the cache
   const bool dsplit = g.D > 256;
   if (dsplit && path == 2) return -2;
-  // the long-window kernel from 65 rows per KV head on.  At head_dim 512 that
-  // is 9 row groups of the VALU kernel: 256 new rows over contexts of 700 to
-  // 3000 (2048 rows per KV head) take 145 us against 314 us.
-  p.prefill = p.NR > 64 && (dsplit ? path == 0 && Lq > 1 : path != 1);
-  p.use_mfma = p.prefill || (!dsplit && (path == 2 || (path == 0 && p.NR > 8)));
-  if (!p.use_mfma && !dsplit && p.NR > 8) return -2;
   const int32_t nb_max = std::max(1, (max_seq_len + 63) / 64);
   const int64_t tmax = (int64_t)B * nb_max;
   const int64_t cus = g.num_cus > 0 ? g.num_cus : 256;
+  // the long-window kernel from 65 rows per KV head on, where its ranges are
+  // long enough (a chosen split: always).  At head_dim 512 that is 9 row groups
+  // of the VALU kernel: 256 new rows over contexts of 700 to 3000 (2048 rows
+  // per KV head) take 143 us against 312 us.
+  p.prefill = p.NR > 64 && (dsplit ? path == 0 && Lq > 1 : path != 1) &&
+              (split_blocks > 0 || long_window_faster(g, B, nb_max, p.NR, cus));
+  p.use_mfma = p.prefill || (!dsplit && (path == 2 || (path == 0 && p.NR > 8)));
+  if (!p.use_mfma && !dsplit && p.NR > 8) return -2;
   if (p.use_mfma) {
     // MFMA: 16 query rows per wave (a row group); the row groups of a KV head
     // go to workgroups of up to 4 waves that share one LDS ring, so a block
@@ -1170,7 +1197,7 @@ int32_t plan_attention(const PoolGeometry &g, int32_t B, int32_t Hq, int32_t Lq,
     // 16-row wave leaves room for two waves per SIMD.
     // 17-32 rows (speculative verify) at D <= 128: one 32-row group per
     // workgroup whose two waves split each block's tokens instead, so no
-    // byte is converted twice.  More than 64 rows (chunked prefill): the
+    // byte is converted twice.  Chunked prefill: the
     // long-window kernel, at D <= 128 with 32-row waves (each LDS read feeds
     // two row tiles) when a batch of max_seq_len sequences gives every
     // workgroup of that grid at least 16 blocks to stream: a 3900-row prompt

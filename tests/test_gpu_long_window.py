@@ -1,7 +1,8 @@
 """Attention of long query windows (more than 64 rows per KV head): the kernel of
 attn_prefill.hip against the fp64 oracle, at the edges of its row tiles (16 and 32 rows a
 wave, four waves a workgroup), of its 64-key blocks, of its 64-entry table window and of the
-block ranges a workgroup takes.
+block ranges a workgroup takes.  A chosen split always runs it; with the automatic one, calls
+over few blocks stay with the verify or decode kernel (test_calls_over_few_blocks).
 
 Bound: bf16 and fp16 inputs reach the matrix cores exactly, the weights as fp16 pairs (2^-22)
 and the sums are binary32, so outputs of values of order 1 lie within 1e-4 of the oracle; 2e-3
@@ -19,10 +20,10 @@ pytestmark = pytest.mark.gpu
 ATOL = 2e-3
 
 
-def _run(mode, D, H, R, lens, Lq, dt="bf16", scale=None, split_blocks=0, out_dtype=torch.float32, q_mul=1.0, seed=0):
+def _run(mode, D, H, R, lens, Lq, dt="bf16", scale=None, split_blocks=1, out_dtype=torch.float32, q_mul=1.0, seed=0):
     rng = np.random.default_rng(seed)
     pool = krill_amd.KVPool(1, H, D, sum((n + 63) // 64 for n in lens) + 4, mode, dt, free_list_seed=7)
-    if split_blocks:
+    if split_blocks:  # (one block a range, if not told otherwise)
         pool.set_option(krill_amd._lib.OPT_SPLIT_BLOCKS, split_blocks)
     f = Filled(pool, lens, rng, dt, max_chunk=500)
     tables, n, _ = f.tables()
@@ -47,7 +48,7 @@ def test_row_and_block_edges(mode, D, R, Lq):
 
 
 @pytest.mark.parametrize("mode", ["affine_g64", "ref_row"])
-@pytest.mark.parametrize("D,split", [(64, 0), (128, 0), (128, 3), (256, 2), (512, 2)])
+@pytest.mark.parametrize("D,split", [(64, 0), (128, 64), (128, 3), (256, 2), (512, 2)])
 def test_ranges_across_sequences(mode, D, split):
     """Ranges that begin and end inside sequences (partials merged), whole sequences inside one
     range, and (automatic split, one KV head) ranges over several sequences."""
@@ -125,6 +126,32 @@ def test_low_precision_output(D, out):
     got, ref = _run("affine_g64", D, 1, 4, [40, 333], 19, out_dtype=out, split_blocks=2, seed=17)
     ulp = 2.0 ** -8 if out is torch.bfloat16 else 2.0 ** -11
     assert (np.abs(got - ref) - ulp * np.abs(ref)).max() <= ATOL
+
+
+@pytest.mark.parametrize("mode,D,H,R,Lq,lens,ranges", [
+    ("affine_g64", 256, 8, 2, 100, [400], 8),       # 7 blocks, at most 1.5 a range: verify kernel, one workgroup a CU
+    ("affine_g64", 256, 8, 2, 200, [500] * 4, 9),   # 32 blocks: this kernel, two
+    ("affine_g64", 256, 8, 2, 40, [40, 33 + 7], 32),  # one block each: this kernel
+    ("ref_row", 256, 8, 2, 100, [190], None),
+    ("ref_row", 256, 8, 2, 100, [420, 100, 333], None),
+    ("affine_g64", 128, 8, 5, 48, [148], None),
+    ("affine_g64", 128, 8, 5, 48, [48], None),
+    ("affine_g64", 128, 8, 5, 60, [160, 60], None),  # more than 4096 rows
+    ("ref_row", 128, 8, 5, 17, [117], None),
+    ("ref_row", 128, 8, 5, 48, [900], None),
+    ("affine_g64", 512, 2, 8, 30, [130, 30], None),  # decode kernel
+    ("affine_g64", 512, 2, 8, 130, [130, 161], None),  # more than 4096 rows, over a quarter block a range
+    ("ref_row", 512, 2, 8, 30, [1030, 700], None),
+])
+def test_calls_over_few_blocks(mode, D, H, R, Lq, lens, ranges):
+    """Either side of each line between this kernel and the one that starts sooner."""
+    print(f"\ncase long_window_few mode={mode} D={D} R={R} Lq={Lq} lens={lens}", flush=True)
+    if ranges is not None:
+        pool = krill_amd.KVPool(1, H, D, 4, mode, "bf16")
+        assert _ranges(pool, len(lens), H * R, Lq, max(lens), 16) == ranges
+        pool.close()
+    got, ref = _run(mode, D, H, R, lens, Lq, split_blocks=0, seed=D + Lq)
+    assert np.abs(got - ref).max() <= ATOL
 
 
 def test_many_query_heads_per_kv_head():
