@@ -1372,13 +1372,17 @@ hipError_t launch_attention_windowed(const PoolGeometry &g, int32_t layer, const
 // 28.8 at 1024), and with ragged lengths the longest sequence decides.  One
 // workgroup fills a compute unit: past one round of them (384 workgroups on
 // 256 units, 128 dims, lengths 10-320) the flat split is faster, 24.2 against
-// 31.2 us.
+// 31.2 us.  Row mode dequantizes every byte: at 256 dims, and at 128 with 6 to 8
+// rows, a wave has no more than one block (256 dims, 2 rows, batch of 4: flat 22.6 against
+// 20.2 us at 450 tokens, 23.2 against 25.6 at 767; 128 dims, 8 rows, batch of 4:
+// 19.2 against 20.4 at 767).
 static bool per_sequence_decode(const PoolGeometry &g, const AttnLaunch &a, const AttnPlan &p) {
   if (p.use_mfma || g.D > 256 || p.split_blocks > 0) return false;
   if (a.window > 0 || a.partial_only || a.len_const >= 0 || !a.causal) return false;
   if (a.rope_cs && (!a.k_new || a.Lq != 1)) return false;
   if ((int64_t)a.B * g.Hkv > g.num_cus) return false;
   const int32_t waves = valu_window_limit(g, p.NR, a.rope_cs != nullptr) / (64 * 64);
+  if (g.mode == MODE_REF && (g.D == 256 || (g.D == 128 && p.NR > 5))) return p.nb_cap <= waves;
   return 2 * p.nb_cap <= 3 * waves;
 }
 

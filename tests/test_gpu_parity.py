@@ -174,9 +174,10 @@ def _attn_case(mode, D, H, R, lens, Lq=1, dt="bf16", split_blocks=0, path=0, out
 
 @pytest.mark.parametrize("mode", ["affine_g64", "ref_row"])
 @pytest.mark.parametrize("D,R", [(128, 5), (64, 4), (128, 8), (256, 2), (128, 1), (512, 8), (512, 1)])
-def test_decode_attention_valu(mode, D, R):
-    print(f"\ncase decode_valu mode={mode} D={D} R={R}", flush=True)
-    got, ref = _attn_case(mode, D, 2, R, [1, 63, 64, 65, 300, 700], seed=D + R)
+@pytest.mark.parametrize("split", [0, 2])  # 0: short sequences, a workgroup each
+def test_decode_attention_valu(mode, D, R, split):
+    print(f"\ncase decode_valu mode={mode} D={D} R={R} split={split}", flush=True)
+    got, ref = _attn_case(mode, D, 2, R, [1, 63, 64, 65, 300, 700], seed=D + R, split_blocks=split)
     err = np.abs(got - ref).max()
     assert err <= ATOL, f"max abs error {err:.3e}"
 
@@ -185,14 +186,17 @@ def test_decode_attention_valu(mode, D, R):
 @pytest.mark.parametrize("D,R,Lq,dt", [(128, 3, 1, "bf16"), (128, 6, 1, "f16"), (128, 7, 1, "bf16"),
                                        (128, 2, 2, "f16"), (128, 1, 3, "bf16"), (128, 2, 3, "bf16"),
                                        (512, 3, 1, "bf16"), (512, 6, 1, "f16")])
-def test_decode_attention_matrix_core_scores_rows(mode, D, R, Lq, dt):
+@pytest.mark.parametrize("split", [0, 2])
+def test_decode_attention_matrix_core_scores_rows(mode, D, R, Lq, dt, split):
     """Every row count of the decode kernel's matrix-core scores (3-8 rows
     per KV head at head_dim 128, 1-8 per row group at 512): the S^T tiles
     carry 16 rows, the rows past R * Lq are zero operands, and the sums go
     back to one token per lane through LDS; short query chunks (Lq > 1) mix
-    causal limits into the rows."""
-    print(f"\ncase decode_msc mode={mode} D={D} R={R} Lq={Lq} dt={dt}", flush=True)
-    got, ref = _attn_case(mode, D, 2, R, [Lq, 63, 64, 65, 300, 700], Lq=Lq, dt=dt, path=1, seed=D + 7 * R + Lq)
+    causal limits into the rows.  At head_dim 128 these lengths run a
+    workgroup per sequence, without those scores, unless a split is chosen."""
+    print(f"\ncase decode_msc mode={mode} D={D} R={R} Lq={Lq} dt={dt} split={split}", flush=True)
+    got, ref = _attn_case(mode, D, 2, R, [Lq, 63, 64, 65, 300, 700], Lq=Lq, dt=dt, path=1, seed=D + 7 * R + Lq,
+                          split_blocks=split)
     err = np.abs(got - ref).max()
     assert err <= ATOL, f"max abs error {err:.3e}"
 
@@ -257,10 +261,11 @@ def test_decode_attention_any_workspace_contents(R):
 
 
 @pytest.mark.parametrize("out_dtype", ["bf16", "f16"])
-def test_decode_attention_low_precision_output(out_dtype):
-    print(f"\ncase decode_out {out_dtype}", flush=True)
+@pytest.mark.parametrize("split", [0, 2])
+def test_decode_attention_low_precision_output(out_dtype, split):
+    print(f"\ncase decode_out {out_dtype} split={split}", flush=True)
     td = torch.bfloat16 if out_dtype == "bf16" else torch.float16
-    got, ref = _attn_case("affine_g64", 128, 2, 5, [77, 300], out_dtype=td, seed=4)
+    got, ref = _attn_case("affine_g64", 128, 2, 5, [77, 300], out_dtype=td, seed=4, split_blocks=split)
     # output rounding (half an ulp of the output dtype) on top of the 2e-3 bound
     ulp = 2.0 ** -8 if out_dtype == "bf16" else 2.0 ** -11
     err = np.abs(got - ref) - 0.5 * ulp * np.maximum(np.abs(ref), 1e-30) * 2
@@ -288,10 +293,13 @@ def test_verify_attention_token_split_partial_rows(mode, D, R, Lq):
     assert err <= ATOL, f"max abs error {err:.3e}"
 
 
-def test_verify_attention_mfma_splits_and_row_groups():
-    print("\ncase verify_mfma_rowgroups", flush=True)
-    # 16 draft rows x 5 heads = 80 rows -> several row groups; small splits
-    got, ref = _attn_case("affine_g64", 128, 2, 5, [40, 300, 777], Lq=16, split_blocks=2, seed=5)
+@pytest.mark.parametrize("Lq,split", [(16, 2), (16, 0), (12, 2), (7, 2)])
+def test_verify_attention_mfma_splits_and_row_groups(Lq, split):
+    """16 draft rows x 5 heads = 80 rows -> several row groups; small splits (the long-window
+    kernel) and the automatic one (few blocks: the verify kernel's groups of four waves); 60 and
+    35 rows: such groups over ranges of two blocks."""
+    print(f"\ncase verify_mfma_rowgroups Lq={Lq} split={split}", flush=True)
+    got, ref = _attn_case("affine_g64", 128, 2, 5, [40, 300, 777], Lq=Lq, split_blocks=split, seed=5)
     err = np.abs(got - ref).max()
     assert err <= ATOL, f"max abs error {err:.3e}"
 
