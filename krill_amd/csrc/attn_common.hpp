@@ -1,4 +1,4 @@
-// Arguments and workspace layout shared by the paged attention kernels
+// Arguments, workspace layout and helpers shared by the paged attention kernels
 // (VALU and MFMA paths).
 #pragma once
 
@@ -217,6 +217,13 @@ __device__ __forceinline__ int64_t out_row_base(const AttnArgs &a, int b, int hk
   const int hq = hk * a.R + r % a.R, j = r / a.R;
   return (((int64_t)b * a.Hq + hq) * a.Lq + j) * D;
 }
+
+// How far (log2 units) a score may exceed the verify and decode kernels' running
+// maximum before it is raised.  Affine mode rounds weights p s_v to fp16: the
+// quantizer's scales are at most 65504 / 127 in magnitude, so with p < 2^6.9 they
+// stay below 61600.  Row mode rounds p alone.
+template <int MODE>
+constexpr float max_rise() { return MODE == MODE_AFFINE ? 6.9f : 8.0f; }
 
 // Inclusive prefix sum over the 64 lanes of a wave.
 __device__ __forceinline__ int wave_incl_scan(int v) {

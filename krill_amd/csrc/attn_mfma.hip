@@ -476,7 +476,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1))) voi
 
       // ---- online softmax with a lazily raised running max (row n of each
       // tile; its 64 scores live in the four lanes n, n+16, n+32, n+48): the
-      // max only moves when some score exceeds it by more than 2^8, so the
+      // max only moves when some score exceeds it by more than max_rise, so the
       // weights stay below 2^8 and most blocks skip the rescale
       float mb[NRT];
       bool over = false;
@@ -489,7 +489,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1))) voi
         v = fmaxf(v, shfl_xor(v, 16));
         v = fmaxf(v, shfl_xor(v, 32));
         mb[rt] = v;
-        over |= v > m_run[rt] + 8.0f;
+        over |= v > m_run[rt] + max_rise<MODE>();
       }
       if (__any(over)) {
 #pragma unroll
@@ -519,7 +519,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(1))) voi
       }
 
       // ---- O^T += V^T . P^T over two 32-token groups; weights p * s_v
-      // (below 2^8 * s_v) as fp16 high and low parts, V bytes as exact fp16
+      // (below 2^6.9 * s_v) as fp16 high and low parts, V bytes as exact fp16
       // u - 128, the zero points (and 128 s_v) summed on the side
 #pragma unroll
       for (int tgi = 0; tgi < NTG; ++tgi) {

@@ -33,7 +33,7 @@
 //    sums return to one token per lane through LDS;
 //  * online softmax in the log2 domain with a lazily raised running max: a
 //    block only pays for a wave reduction when some score exceeds the
-//    running max by more than 8 (a wave vote), so weights stay below 2^8;
+//    running max by more than max_rise (a wave vote), so weights stay below 2^8;
 //  * weights w = p * s_v (binary32) go to LDS in V storage order, and P.V
 //    runs on the matrix cores: O^T += V^T . P^T per 16-row d tile with
 //    v_mfma_f32_16x16x32_f16, A = the V bytes as exact fp16 (u - 128; row
@@ -980,7 +980,7 @@ __global__ __launch_bounds__(64 * (seq_waves<D, NR, MODE, VAR>() > 0 ? seq_waves
     if (!raise) {
       bool over = false;
 #pragma unroll
-      for (int r = 0; r < NR; ++r) over |= s[r] > m_run[r] + 8.0f;
+      for (int r = 0; r < NR; ++r) over |= s[r] > m_run[r] + max_rise<MODE>();
       raise = __any(over);
     }
     if (raise) {

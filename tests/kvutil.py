@@ -76,6 +76,41 @@ class Filled:
         return kq, ks, kz, vq, vs, vz
 
 
+class Rising(Filled):
+    """Scores that rise by `rise` log2 units a block (at scale ln 2) over V groups spanning
+    -64000 .. 65504, or (s_v > 0) V scales of that size brought in through scatter.  Row mode
+    stores f16(max - min) / 255, so its rows span -32000 .. 32704: past 65504 the stored scale
+    is infinite by definition."""
+
+    def __init__(self, pool, lens, rng, rise, s_v=0.0):
+        import torch
+
+        self.pool, self.lens, self.dt, H, D = pool, list(lens), "f16", pool.num_kv_heads, pool.head_dim
+        self.mode, self.snap = MODE[pool.quant_mode], {}
+        self.seqs = [pool.seq_create() for _ in lens]
+        for b, T in enumerate(lens):
+            k = rng.standard_normal((1, H, T, D)).astype(np.float32) * 0.01
+            k[..., 0] = rise * (np.arange(T) // 64)
+            v_lo, v_hi = (-64000, 65504) if self.mode == MODE["affine_g64"] else (-32000, 32704)
+            v = rng.uniform(v_lo, v_hi, (1, H, T, D)).astype(np.float32)
+            v[..., 0::64], v[..., 1::64] = v_lo, v_hi
+            slots = i32(pool.reserve_append(self.seqs[b], T).reshape(1, T))
+            pool.quantize_append(0, to_dev(O.f32_to_f16_bits(k), "f16"), to_dev(O.f32_to_f16_bits(v), "f16"), slots)
+            t, n = pool.batch_tables([self.seqs[b]], (T + 63) // 64)
+            s = pool.gather(0, i32(t), i32(n), T)
+            if s_v:
+                s["value_scales"].copy_(torch.from_numpy(rng.uniform(-s_v, s_v, s["value_scales"].shape)).half())
+                s["value_zeros"].zero_()
+                pool.scatter(0, s, i32([0]), slots)
+            self.snap[b] = s
+
+    def expected(self, layer, b):
+        g = {n: x[0].cpu().numpy() for n, x in self.snap[b].items()}
+        bits = lambda x: x.view(np.uint16)  # noqa: E731
+        return (g["keys"], bits(g["key_scales"]), bits(g["key_zeros"]),
+                g["values"], bits(g["value_scales"]), bits(g["value_zeros"]))
+
+
 def oracle_attention(pool, filled: Filled, layer: int, q_bits: np.ndarray, dt: str, scale: float):
     """Reference outputs [B, Hq, Lq, D] (float64) for q_bits [B, Hq, Lq, D]."""
     B, Hq, Lq, D = q_bits.shape

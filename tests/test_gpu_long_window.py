@@ -14,7 +14,7 @@ torch = pytest.importorskip("torch")
 
 import krill_amd  # noqa: E402
 from oracle import oracle as O  # noqa: E402
-from tests.kvutil import MODE, Filled, i32, oracle_attention, rand_bits, to_dev  # noqa: E402
+from tests.kvutil import Filled, Rising, i32, oracle_attention, rand_bits, to_dev  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 ATOL = 2e-3
@@ -190,39 +190,6 @@ def test_blocks_at_the_pools_end():
     assert np.abs(got.double().cpu().numpy() - ref).max() <= ATOL
 
 
-class _Rising(Filled):
-    """Scores that rise by `rise` log2 units a block (at scale ln 2) over V groups spanning
-    -64000 .. 65504, or (s_v > 0) V scales of that size brought in through scatter.  Row mode
-    stores f16(max - min) / 255, so its rows span -32000 .. 32704: past 65504 the stored scale
-    is infinite by definition."""
-
-    def __init__(self, pool, lens, rng, rise, s_v=0.0):
-        self.pool, self.lens, self.dt, H, D = pool, list(lens), "f16", pool.num_kv_heads, pool.head_dim
-        self.mode, self.snap = MODE[pool.quant_mode], {}
-        self.seqs = [pool.seq_create() for _ in lens]
-        for b, T in enumerate(lens):
-            k = rng.standard_normal((1, H, T, D)).astype(np.float32) * 0.01
-            k[..., 0] = rise * (np.arange(T) // 64)
-            v_lo, v_hi = (-64000, 65504) if self.mode == MODE["affine_g64"] else (-32000, 32704)
-            v = rng.uniform(v_lo, v_hi, (1, H, T, D)).astype(np.float32)
-            v[..., 0::64], v[..., 1::64] = v_lo, v_hi
-            slots = i32(pool.reserve_append(self.seqs[b], T).reshape(1, T))
-            pool.quantize_append(0, to_dev(O.f32_to_f16_bits(k), "f16"), to_dev(O.f32_to_f16_bits(v), "f16"), slots)
-            t, n = pool.batch_tables([self.seqs[b]], (T + 63) // 64)
-            s = pool.gather(0, i32(t), i32(n), T)
-            if s_v:
-                s["value_scales"].copy_(torch.from_numpy(rng.uniform(-s_v, s_v, s["value_scales"].shape)).half())
-                s["value_zeros"].zero_()
-                pool.scatter(0, s, i32([0]), slots)
-            self.snap[b] = s
-
-    def expected(self, layer, b):
-        g = {n: x[0].cpu().numpy() for n, x in self.snap[b].items()}
-        bits = lambda x: x.view(np.uint16)  # noqa: E731
-        return (g["keys"], bits(g["key_scales"]), bits(g["key_zeros"]),
-                g["values"], bits(g["value_scales"]), bits(g["value_zeros"]))
-
-
 @pytest.mark.parametrize("mode", ["affine_g64", "ref_row"])
 @pytest.mark.parametrize("D,split", [(64, 64), (128, 64), (128, 3), (256, 64), (512, 64), (512, 2)])
 @pytest.mark.parametrize("rise,s_v", [(2.1, 0), (2.5, 0), (2.9, 0), (7.5, 0), (0.0, 3000.0), (2.9, 60000.0)])
@@ -239,7 +206,7 @@ def test_large_value_scales(mode, D, split, rise, s_v):
     R, Lq, lens = 5, 20, [600, 40, 64 * 4]
     pool = krill_amd.KVPool(1, 1, D, 24, mode, "f16", free_list_seed=5)
     pool.set_option(krill_amd._lib.OPT_SPLIT_BLOCKS, split)
-    f = _Rising(pool, lens, rng, rise, s_v)
+    f = Rising(pool, lens, rng, rise, s_v)
     tables, n, _ = f.tables()
     q = rng.standard_normal((len(lens), R, Lq, D)).astype(np.float32) * 0.01
     q[..., 0] = 1.0

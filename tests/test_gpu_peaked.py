@@ -14,7 +14,7 @@ Gemma4Model.swift:516-517)."""
 import numpy as np
 import pytest
 
-from kvutil import DT, MODE, Filled, oracle_attention, to_dev
+from kvutil import DT, MODE, Filled, Rising, oracle_attention, to_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -182,3 +182,31 @@ def test_fused_append_of_a_dominant_token(mode):
     print(f"max abs error {err:.3e}", flush=True)
     pool.close()
     assert err <= ATOL, f"max abs error {err:.3e}"
+
+
+@pytest.mark.parametrize("mode", ["affine_g64", "ref_row"])
+@pytest.mark.parametrize("D,R,Lq,path", [(64, 4, 1, 0), (128, 5, 1, 0), (128, 1, 1, 0), (256, 2, 1, 0), (512, 8, 1, 0),
+                                         (128, 5, 1, 2), (64, 5, 8, 0), (128, 4, 8, 0), (128, 5, 8, 0), (256, 2, 8, 0),
+                                         (512, 2, 3, 0)])
+@pytest.mark.parametrize("rise", [2.9, 6.95, 7.5])
+def test_large_value_scales(mode, D, R, Lq, path, rise):
+    """Decode and verify: weights p s_v stay finite in fp16 while scores rise without raising the
+    running maximum, over V groups spanning all of fp16 (long query windows: the long-window
+    test of this name, whose bound this is: 2^-14 of the largest |V|)."""
+    print(f"\ncase large_v mode={mode} D={D} R={R} Lq={Lq} path={path} rise={rise}", flush=True)
+    rng = np.random.default_rng(37)
+    lens = [900, 40, 64 * 4]
+    pool = krill_amd.KVPool(1, 1, D, 24, mode, "f16", free_list_seed=5)
+    pool.set_option(krill_amd._lib.OPT_SPLIT_BLOCKS, 16)
+    pool.set_option(krill_amd._lib.OPT_ATTN_PATH, path)
+    f = Rising(pool, lens, rng, rise)
+    tables, n, _ = f.tables()
+    q = rng.standard_normal((len(lens), R, Lq, D)).astype(np.float32) * 0.01
+    q[..., 0] = 1.0
+    q = O.f32_to_f16_bits(q)
+    got = pool.attention(0, to_dev(q, "f16"), tables, n, max(lens), float(np.log(2.0)), torch.float32)
+    got = got.double().cpu().numpy()
+    ref = oracle_attention(pool, f, 0, q, "f16", float(np.log(2.0)))
+    pool.close()
+    assert np.isfinite(got).all()
+    assert np.abs(got - ref).max() <= 2.0 ** -14 * 65504
