@@ -218,3 +218,67 @@ def test_large_value_scales(mode, D, split, rise, s_v):
     top = max(255 * s_v, 65504.0)
     assert np.isfinite(got).all()
     assert np.abs(got - ref).max() <= 2.0 ** -14 * top
+
+
+@pytest.mark.parametrize("mode", ["affine_g64", "ref_row"])
+@pytest.mark.parametrize("D,H,R,Lq", [(64, 2, 4, 342), (128, 2, 5, 280), (256, 2, 2, 690), (512, 1, 8, 350)])
+def test_merge_by_row_groups(mode, D, H, R, Lq):
+    """From 8192 rows the partials are merged by row group: 72 partials of a sequence (more than
+    a wave reads at once), few, and a sequence with no blocks, whose rows are zero.  Against the
+    same sequences one by one, below 8192 rows each, merged by row: the same partials, at most 72
+    binary32 terms under 4 summed in another order."""
+    print(f"\ncase long_window_merge mode={mode} D={D}", flush=True)
+    rng = np.random.default_rng(41)
+    lens = [72 * 64 - 5, Lq + 3, 0, Lq]
+    assert 4 * H * R * Lq >= 8192 > H * R * Lq
+    pool = krill_amd.KVPool(1, H, D, sum((T + 63) // 64 for T in lens) + 4, mode, "bf16", free_list_seed=9)
+    pool.set_option(krill_amd._lib.OPT_SPLIT_BLOCKS, 1)
+    f = Filled(pool, lens, rng, "bf16", max_chunk=4000)
+    tables, n, _ = f.tables()
+    q = to_dev(rand_bits(rng, (len(lens), H * R, Lq, D), "bf16"), "bf16")
+    got = pool.attention(0, q, tables, n, max(lens), 1.0 / np.sqrt(D))
+    for b in range(len(lens)):
+        one = pool.attention(0, q[b:b + 1], tables[b:b + 1], n[b:b + 1], max(lens), 1.0 / np.sqrt(D))
+        assert (got[b] - one[0]).abs().max() <= 72 * 2.0 ** -24 * 4
+    assert not got[2].any()
+    # and rows of the first against the decode kernel (two kernels, each within 1e-4 of fp64)
+    want = pool.attention(0, q[:1, :, Lq - 1:].contiguous(), tables[:1], n[:1], max(lens), 1.0 / np.sqrt(D))
+    assert (got[:1, :, Lq - 1:] - want).abs().max() <= 2e-4
+    pool.close()
+
+
+@pytest.mark.parametrize("mode", ["affine_g64", "ref_row"])
+@pytest.mark.parametrize("D,H,R,lens,split", [(64, 2, 70, [70, 1, 200, 64], 2), (128, 2, 70, [70, 1, 200, 64], 2),
+                                              (256, 2, 72, [517, 63], 3), (64, 8, 1024, [1000] * 8, 0),
+                                              (128, 8, 1024, [1000] * 8, 0)])
+def test_rope_step_of_many_query_heads(mode, D, H, R, lens, split):
+    """The fused decode step with RoPE of 65 and more query heads per KV head (16-row waves, and
+    32-row ones): the RoPE append, then attention of queries rotated by the oracle, bit for bit."""
+    print(f"\ncase long_window_rope mode={mode} D={D} R={R}", flush=True)
+    B, dt, scale = len(lens), "bf16", 1.0 / np.sqrt(D)
+    rng = np.random.default_rng(D + R)
+    kn, vn = rand_bits(rng, (B, H, 1, D), dt), rand_bits(rng, (B, H, 1, D), dt)
+    q = rand_bits(rng, (B, H * R, 1, D), dt)
+    pos = np.array(lens, np.int32)
+    full, mx = [T + 1 for T in lens], max(lens) + 1
+    cs = krill_amd.pool.rope_table(mx, D)
+    csd = torch.from_numpy(cs).cuda()
+    outs, snaps = [], []
+    for fused in (False, True):
+        pool = krill_amd.KVPool(1, H, D, sum((T + 63) // 64 for T in full) + 4, mode, dt, free_list_seed=3)
+        pool.set_option(krill_amd._lib.OPT_SPLIT_BLOCKS, split)
+        f = Filled(pool, lens, np.random.default_rng(7), dt, max_chunk=300)
+        slots = np.stack([pool.reserve_append(s, 1).copy() for s in f.seqs])
+        tables, n = (i32(a) for a in pool.batch_tables(f.seqs, (mx + 63) // 64))
+        if fused:
+            outs.append(pool.decode_append_attention_rope(0, to_dev(q, dt), to_dev(kn, dt), to_dev(vn, dt), tables, n,
+                                                          mx, scale, csd))
+        else:
+            pool.quantize_append_rope(0, to_dev(kn, dt), to_dev(vn, dt), i32(slots), i32(pos.reshape(B, 1)), csd)
+            q_rot = O.rope_rows(q, O.DT_BF16, np.broadcast_to(pos[:, None, None], (B, H * R, 1)), cs)
+            outs.append(pool.attention(0, to_dev(q_rot, dt), tables, n, mx, scale))
+        snaps.append({k: v.cpu() for k, v in pool.gather(0, tables, n, mx).items()})
+        pool.close()
+    assert torch.equal(outs[0], outs[1])
+    for k in snaps[0]:
+        assert torch.equal(snaps[0][k].view(torch.uint8), snaps[1][k].view(torch.uint8)), k

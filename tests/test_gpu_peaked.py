@@ -77,12 +77,13 @@ def _top_mass(pool, f, q_bits, dt, scale, Lq, R, k=3):
     return worst
 
 
-def _case(mode, variant, Lq, path, seed, dt="bf16"):
+def _case(mode, variant, Lq, path, seed, dt="bf16", split=0):
     H, R, D = 2, (5 if Lq == 1 else 4), 128
     lens = [700, 2100] if Lq == 1 else [1100, 2500]
     rng = np.random.default_rng(seed)
     pool = krill_amd.KVPool(1, H, D, sum((T + 63) // 64 for T in lens) + 8, mode, dt, free_list_seed=seed)
     pool.set_option(krill_amd._lib.OPT_ATTN_PATH, path)
+    pool.set_option(krill_amd._lib.OPT_SPLIT_BLOCKS, split)
     outl = 0.01 if variant == "three_keys_outliers" else 0.0
     f = Filled(pool, lens, rng, dt, outlier_frac=outl)
     tables, tl, _ = f.tables()
@@ -119,6 +120,18 @@ def test_decode_valu_peaked(mode, variant):
 def test_verify_mfma_peaked(mode, variant):
     print(f"\ncase peaked verify_mfma mode={mode} variant={variant}", flush=True)
     got, ref, mass = _case(mode, variant, 8, 0, seed=400 + VARIANTS.index(variant))
+    assert mass > MIN_MASS[variant], f"softmax not peaked: top-3 mass {mass:.4f}"
+    err = np.abs(got - ref).max()
+    print(f"max abs error {err:.3e} (top-3 mass >= {mass:.4f})", flush=True)
+    assert err <= ATOL, f"max abs error {err:.3e}"
+
+
+@pytest.mark.parametrize("variant", VARIANTS)
+@pytest.mark.parametrize("mode", ["affine_g64", "ref_row"])
+def test_long_window_peaked(mode, variant):
+    """96 rows per KV head, 8 blocks a range: the long-window kernel."""
+    print(f"\ncase peaked long_window mode={mode} variant={variant}", flush=True)
+    got, ref, mass = _case(mode, variant, 24, 0, seed=600 + VARIANTS.index(variant), split=8)
     assert mass > MIN_MASS[variant], f"softmax not peaked: top-3 mass {mass:.4f}"
     err = np.abs(got - ref).max()
     print(f"max abs error {err:.3e} (top-3 mass >= {mass:.4f})", flush=True)

@@ -158,6 +158,26 @@ def test_window_chunk_parity(mode):
         p.close()
 
 
+@pytest.mark.parametrize("mode", ["affine_g64", "ref_row"])
+@pytest.mark.parametrize("D,R,Lq", [(128, 4, 40), (256, 2, 33), (256, 2, 70), (512, 8, 9), (512, 8, 70)])
+def test_window_chunk_long_rows(mode, D, R, Lq):
+    """More than 64 rows per KV head (65 to 560) on the long-window kernel, two blocks a range:
+    rows whose windows start in different blocks, a window reaching back past one range."""
+    print(f"\ncase window_long_rows mode={mode} D={D} Lq={Lq}", flush=True)
+    W, H = 100, 2
+    rng = np.random.default_rng(D + Lq)
+    pools = _pools(mode, H, D, 64, W, seed=D)
+    sl = [Seqs(p, 3, 600, np.random.default_rng(45)) for p in pools]
+    for p, ss in zip(pools, sl):
+        p.set_option(krill_amd._lib.OPT_SPLIT_BLOCKS, 2)
+        for b, T in enumerate([300, 90, 5]):
+            ss.append(b, T)
+            ss.append(b, Lq)
+    _check(pools, sl, W, Lq, mode, rng, R, tol_pair=1e-3)
+    for p in pools:
+        p.close()
+
+
 def test_window_truncate_then_decode():
     """After a rollback inside the retained tail the first retained token
     binds (fewer than window keys visible), as in RotatingKVCacheTests
