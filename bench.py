@@ -1187,8 +1187,8 @@ def run_verify(args, w):
     compute_bound = ai > MFMA_F16_PEAK_TFLOPS * 1e12 / (HBM_PEAK_GBS * 1e9)  # above the ridge (~312 FLOP/B)
     roofline = {
         "bound": "mfma" if compute_bound else "hbm",
-        "kernel": ("chunked-prefill" if not rollback else "verify") + " attention call (k_attn_mfma + "
-                  "k_attn_merge_flat), one layer",
+        "kernel": ("verify attention call (k_attn_mfma + k_attn_merge_flat), one layer" if rollback
+                   else "chunked-prefill attention call (k_attn_prefill + k_attn_merge_rows), one layer"),
         "achieved": mfma["achieved"] if compute_bound else hbm["achieved"],
         "peak": MFMA_F16_PEAK_TFLOPS if compute_bound else HBM_PEAK_GBS,
         "unit": "TFLOP/s" if compute_bound else "GB/s",

@@ -23,11 +23,12 @@
 //    fma);
 //  * weights p * s_v are split into fp16 high and low parts in three full-rate
 //    instructions each, alternating with the products of the step before.
-// Measured, calls with their append (the verify kernel, or at head_dim 512 the
-// decode kernel, before): 8 x 512 rows on contexts of 2048-6144, Hq 40, D 128:
-// 762 us = 479 TFLOP/s (1073); a 3900-row prompt, row mode, Hq 32: 240 us = 520
-// TFLOP/s (533); 2 x 256 rows at head_dim 512: 134 us (288); 4 x 512 rows,
-// window 1024, head_dim 256: 162 us (298).
+// Measured on one card, calls with their append (the verify kernel, or at
+// head_dim 512 the decode kernel, before): 8 x 512 rows on contexts of
+// 2048-6144, Hq 40, D 128: 789 us = 463 TFLOP/s (1108); a 3900-row prompt, row
+// mode, Hq 32: 242 us = 515 TFLOP/s (534); 2 x 256 rows at head_dim 512: 145 us
+// (310); 4 x 512 rows, window 1024, head_dim 256: 169 us (304).  Other cards
+// differ by up to 5 %.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>

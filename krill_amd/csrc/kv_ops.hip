@@ -1185,7 +1185,7 @@ int32_t plan_attention(const PoolGeometry &g, int32_t B, int32_t Hq, int32_t Lq,
   // the long-window kernel from 65 rows per KV head on, where its ranges are
   // long enough (a chosen split: always).  At head_dim 512 that is 9 row groups
   // of the VALU kernel: 256 new rows over contexts of 700 to 3000 (2048 rows
-  // per KV head) take 143 us against 312 us.
+  // per KV head) take 145 us against 310 us.
   p.prefill = p.NR > 64 && (dsplit ? path == 0 && Lq > 1 : path != 1) &&
               (split_blocks > 0 || long_window_faster(g, B, nb_max, p.NR, cus));
   p.use_mfma = p.prefill || (!dsplit && (path == 2 || (path == 0 && p.NR > 8)));
@@ -1200,11 +1200,12 @@ int32_t plan_attention(const PoolGeometry &g, int32_t B, int32_t Hq, int32_t Lq,
     // byte is converted twice.  Chunked prefill: the
     // long-window kernel, at D <= 128 with 32-row waves (each LDS read feeds
     // two row tiles) when a batch of max_seq_len sequences gives every
-    // workgroup of that grid at least 16 blocks to stream: a 3900-row prompt
-    // takes 265 us so against 332 us with 16-row waves, the cascade over a
-    // shared prefix of 65 blocks, whose 16-row grid keeps more workgroups
-    // busy, 67 against 63 us.  head_dim 256 in 32-row waves, one a SIMD: 172
-    // against 166 us (512 rows, window 1024).
+    // workgroup of that grid at least 16 blocks to stream: 8 x 512 rows on
+    // 2048-6144 tokens take 764 us so against 937 with 16-row waves, a 3900-row
+    // prompt 243 against 271; the cascade over a shared prefix of 64 blocks,
+    // whose 16-row grid keeps more workgroups busy, 68.5 against 65.  head_dim
+    // 256 in 32-row waves, one a SIMD, took 172 against 166 us (512 rows,
+    // window 1024) and is not built.
     p.token_split = 1;
     if (p.prefill) {
       const int64_t grp32 = ((p.NR + 31) / 32 + 3) / 4;
@@ -1281,8 +1282,11 @@ hipError_t launch_attn_merge(const PoolGeometry &g, int32_t layer, const AttnLau
                              hipStream_t st) {
   if (a.B == 0) return hipSuccess;
   const AttnArgs args = make_attn_args(g, layer, a, p);
-  // (few rows: one wave each, side by side -- 2 x 48 new rows, 3072 waves: the
-  // call takes 1 us less so; from 8192 on the workgroups are what costs)
+  // (few rows: one wave each, side by side; from 8192 on their workgroups are
+  // what costs.  Whole calls by row groups over by rows, 693 of them: at 4096
+  // rows 1.12 / 1.10 / 1.04 / 1.05 at head_dim 64 / 128 / 256 / 512, at 6144 1.07
+  // / 1.05 / 1.03 / 1.03, at 8192 0.99 / 0.99 / 1.01 / 1.01, at 12288 0.91 / 0.92 /
+  // 0.98 / 0.98, at 32768 0.78 / 0.81 / 0.89 / 0.96)
   if (p.prefill && (int64_t)p.NR * g.Hkv * a.B >= 8192) {
     const dim3 rows((unsigned)p.row_groups, (unsigned)g.Hkv, (unsigned)a.B);
     KRILL_DISPATCH_D(g.D, { k_attn_merge_rows<D><<<rows, dim3(256), 0, st>>>(args); });
@@ -1370,12 +1374,14 @@ hipError_t launch_attention_windowed(const PoolGeometry &g, int32_t layer, const
 // the two meet (128 dims, 5 rows, 1024 tokens, batch of 4: 22.0 against 22.4;
 // 8 rows, whose LDS leaves 4 waves: 24.2 against 22.9 at 512, 24.7 against
 // 28.8 at 1024), and with ragged lengths the longest sequence decides.  One
-// workgroup fills a compute unit: past one round of them (384 workgroups on
-// 256 units, 128 dims, lengths 10-320) the flat split is faster, 24.2 against
-// 31.2 us.  Row mode dequantizes every byte: at 256 dims, and at 128 with 6 to 8
-// rows, a wave has no more than one block (256 dims, 2 rows, batch of 4: flat 22.6 against
-// 20.2 us at 450 tokens, 23.2 against 25.6 at 767; 128 dims, 8 rows, batch of 4:
-// 19.2 against 20.4 at 767).
+// workgroup fills a compute unit, so at one more than a round of them the call
+// takes this form 1.1 to 1.4 times as long as the flat split (264 workgroups, 64
+// to 256 dims, 40 to 512 tokens, both modes; at 256 the ratios above hold), at 520
+// 1.2 to 1.8 times.  (8 rows of 128 dims in affine mode fit twice: there it stays
+// faster up to 512 workgroups, 0.7 to 0.85.)  Row mode dequantizes every byte: at
+// 256 dims, and at 128 with 6 to 8 rows, a wave has no more than one block (256
+// dims, 2 rows, batch of 4: flat 22.6 against 20.2 us at 450 tokens, 23.2 against
+// 25.6 at 767; 128 dims, 8 rows: 19.2 against 20.4 at 767).
 static bool per_sequence_decode(const PoolGeometry &g, const AttnLaunch &a, const AttnPlan &p) {
   if (p.use_mfma || g.D > 256 || p.split_blocks > 0) return false;
   if (a.window > 0 || a.partial_only || a.len_const >= 0 || !a.causal) return false;
